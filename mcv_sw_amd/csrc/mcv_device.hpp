@@ -296,8 +296,9 @@ __device__ __forceinline__ double riemann(double fxL, double fxR, double qxL, do
 }
 
 // Largest gravity-wave speed along one direction (spatial_operators_mod.F90:248-280)
-__device__ __forceinline__ double wave_speed(double c, double phi, double gii) {
-  double l1 = c - sqrt(gii * phi), l2 = c + sqrt(gii * phi);
+// from the contravariant wind c and gp = IG_ii * phi
+__device__ __forceinline__ double wave_speed(double c, double gp) {
+  const double l1 = c - sqrt(gp), l2 = c + sqrt(gp);
   // the larger of two non-negative values (both NaN together or neither)
   return fmax(fabs(l1), fabs(l2));
 }

@@ -173,16 +173,11 @@ __device__ __forceinline__ void stage_tile_f32(const MeshF32 &m, const StageArgs
       if (inx && iny) {
         const int ox = lx - H, oy = ly - H;
         lds.sSG[TL::core_at(lx, ly)] = rsg[q];
-        const C phi = (C)((double)pg / rsg[q]);  // for the wave speeds only
+        // phase 1 forms the wave speeds (one division and square root per cell
+        // end there, two and four per thread here)
         const int cx = div_small<H>(ox), cy = div_small<H>(oy);
-        if (ox == cx * H) {
-          const C sq = sqrt((C)g11 * phi);
-          lamx[cx * NY + oy] = fmax(fabs(cu - sq), fabs(cu + sq));
-        }
-        if (oy == cy * H) {
-          const C sq = sqrt((C)g22 * phi);
-          lamy[cy * NX + ox] = fmax(fabs(cv - sq), fabs(cv + sq));
-        }
+        if (ox == cx * H) lamx[cx * NY + oy] = (C)g11;
+        if (oy == cy * H) lamy[cy * NX + ox] = (C)g22;
       }
     }
   }
@@ -203,8 +198,12 @@ __device__ __forceinline__ void stage_tile_f32(const MeshF32 &m, const StageArgs
     const int cb = isx ? TL::cu_at(H + mb * H, o + H) : TL::cv_at(o + H, H + mb * H);
     const C *sQ = isx ? sU : sV;
     const C *sW = isx ? sV : sU;
-    const C lam = isx ? lamx[tt] : lamy[tt];
     const C c = sC[cb];
+    // wave speed; phi to FP32 from phiG and the FP64 sqrtG
+    const C phi =
+        (C)((double)sPG[b] / lds.sSG[isx ? o * NX + mb * H : mb * H * NX + o]);
+    const C sq = sqrt((isx ? lamx[tt] : lamy[tt]) * phi);
+    const C lam = fmax(fabs(c - sq), fabs(c + sq));
     const C up = c == C(0) ? C(1) : copysign(C(1), c);
     // the three flux pairs one after the other (only one pair's windows live)
     C fF, fD, fW;

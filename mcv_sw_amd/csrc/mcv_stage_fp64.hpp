@@ -2,9 +2,10 @@
 //
 // Phase 0 stages the cross-shaped tile plus its one-cell halo of (phi, u, v)
 // in LDS together with the derived E = phi + phi_s + K, phiG = phi*sqrtG and
-// the contravariant winds, and the wave speeds at cell ends.  Phase 1 computes
-// the Riemann derivative at every cell end of the tile once (the reference
-// computes each interface twice, from both cells).  Phase 2 forms the
+// the contravariant winds, and the squared gravity-wave speeds IG_ii*phi at cell
+// ends.  Phase 1 computes the wave speed and the Riemann derivative at every
+// cell end of the tile once (the reference computes each interface twice, from
+// both cells).  Phase 2 forms the
 // interior-point derivatives, the vorticity/Coriolis tendencies and the RK
 // update, and writes the raw updated interior plus a raw copy of the H+1
 // lines nearest each panel side (the band) for the boundary pass.  Every loop runs over compile-time
@@ -31,8 +32,9 @@ struct TileLayout {
   static constexpr int kEy = (CY + 1) * NX;  // y-sweep: (CY+1) per core column
   // The contravariant winds are read only along their own sweep: contraU on
   // the core rows (NY x TX), contraV on the core columns (TY x NX).  The
-  // cell-end wave speeds share the storage of the first flux of their sweep:
-  // each phase-1 task reads its wave speed before it writes that flux.
+  // cell-end values the wave speeds are formed from share the storage of the
+  // first flux of their sweep: each phase-1 task reads its own before it
+  // writes that flux.
   static constexpr int kCU = NY * TX, kCV = TY * NX;
   // sqrtG at the core points (FP64 whatever T is), staged for phase 2
   static constexpr int kCore = NX * NY;
@@ -149,8 +151,11 @@ __device__ __forceinline__ void stage_tile(const MeshDev &m, const StageArgs &a,
       if (inx && iny) {
         const int ox = lx - H, oy = ly - H;
         lds.sSG[TL::core_at(lx, ly)] = rsg[q];
-        if (ox % H == 0) lamx[(ox / H) * NY + oy] = wave_speed(cu, phi, g11);
-        if (oy % H == 0) lamy[(oy / H) * NX + ox] = wave_speed(cv, phi, g22);
+        // the wave speed's square root is left to phase 1, whose lanes are all
+        // cell ends (one per thread there; here four, with most lanes idle:
+        // MCV4 6x96^2 90.7 -> 88.9 us, 6x384^2 1078 -> 1070 us per RK4 step)
+        if (ox % H == 0) lamx[(ox / H) * NY + oy] = g11 * phi;
+        if (oy % H == 0) lamy[(oy / H) * NX + ox] = g22 * phi;
       }
     }
   }
@@ -172,8 +177,9 @@ __device__ __forceinline__ void stage_tile(const MeshDev &m, const StageArgs &a,
     const int cb = isx ? TL::cu_at(H + mb * H, o + H) : TL::cv_at(o + H, H + mb * H);
     const double *sQ = isx ? sU : sV;   // q of the gradient flux
     const double *sW = isx ? sV : sU;   // upwinded cross wind
-    const double lam = isx ? lamx[tt] : lamy[tt];
-    const double up = upwind_sign(sC[cb]);
+    const double cb0 = sC[cb];
+    const double lam = wave_speed(cb0, isx ? lamx[tt] : lamy[tt]);
+    const double up = upwind_sign(cb0);
     // the three flux pairs one after the other, each from its own LDS reads,
     // so that only one pair's windows are live at a time
     double fF, fD, fW;
