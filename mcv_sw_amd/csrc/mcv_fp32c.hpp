@@ -248,8 +248,9 @@ __device__ __forceinline__ void stage_tile_f32(const MeshF32 &m, const StageArgs
   }
   __syncthreads();
 
-  // global loads of all a thread's points first, then their LDS work
-  constexpr int kCells = CX * CY, kSlots = H * H * kCells, kTail = NY + NX - 1;
+  // owned points row by row (see stage_tile); global loads of all a thread's
+  // points first, then their LDS work
+  constexpr int kRow = CX * H, kSlots = kRow * CY * H, kTail = NY + NX - 1;
   constexpr int kP2 = (kSlots + kTail + kStageThreads - 1) / kStageThreads;
   const bool first = kind == kRK4S1 || kind == kRK3S1;
   const bool need_in = first || kind == kRK3S2 || kind == kRK3S3;
@@ -268,12 +269,9 @@ __device__ __forceinline__ void stage_tile_f32(const MeshF32 &m, const StageArgs
       int ox = 0, oy = 0;
       bool ok = false;
       if (t < kSlots) {
-        const int cls = div_small<kCells>(t), cell = t - cls * kCells;
-        const int cyl = div_small<CX>(cell), cxl = cell - cyl * CX;
-        const int cly = div_small<H>(cls);
-        ok = cxl < ncx && cyl < ncy;
-        ox = cxl * H + (cls - cly * H);
-        oy = cyl * H + cly;
+        oy = div_small<kRow>(t);
+        ox = t - oy * kRow;
+        ok = ox < ncx * H && oy < ncy * H;
       } else if (t < kSlots + NY) {
         oy = t - kSlots;
         ox = ncx * H;

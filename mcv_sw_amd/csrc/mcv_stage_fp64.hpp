@@ -225,13 +225,17 @@ __device__ __forceinline__ void stage_tile(const MeshDev &m, const StageArgs &a,
   __syncthreads();
 
   // Phase 2: derivatives at owned points, tendencies, RK update.  Points are
-  // visited class by class (position within the cell in x and in y), cells
-  // fastest, so the lanes of a wave take the same branches and read LDS with
-  // a stride of H points (no bank conflicts); the far cell-end column and row
-  // owned by the last tiles follow.
+  // visited row by row, so that the loads and stores of a wavefront cover
+  // whole stretches of each line: with the points class by class (one position
+  // within the cell after the other, for uniform branches) every cache line of
+  // the base state, the accumulator and the output was touched by DOF-1
+  // wavefronts, and the L1 tag look-ups (66 million a launch at MCV4 6x384^2,
+  // 49 million row by row) held the kernel up: 1078 -> 1027 us per RK4 step,
+  // FP32C 811 -> 766.  The far cell-end column and row owned by the last tiles
+  // follow.
   // The global loads of all a thread's points are issued before their LDS
   // work.
-  constexpr int kCells = CX * CY, kSlots = H * H * kCells, kTail = NY + NX - 1;
+  constexpr int kRow = CX * H, kSlots = kRow * CY * H, kTail = NY + NX - 1;
   constexpr int kP2 = (kSlots + kTail + kStageThreads - 1) / kStageThreads;
   const bool need_base = !(kind == kTend || kind == kRK4S1 || kind == kRK3S1);
   const bool need_acc = kind == kRK4S2 || kind == kRK4S3 || kind == kRK4S4;
@@ -246,11 +250,9 @@ __device__ __forceinline__ void stage_tile(const MeshDev &m, const StageArgs &a,
       int ox = 0, oy = 0;
       bool ok = false;
       if (t < kSlots) {
-        const int cls = t / kCells, cell = t - cls * kCells;
-        const int cyl = cell / CX, cxl = cell - cyl * CX;
-        ok = cxl < ncx && cyl < ncy;
-        ox = cxl * H + cls % H;
-        oy = cyl * H + cls / H;
+        oy = t / kRow;
+        ox = t - oy * kRow;
+        ok = ox < ncx * H && oy < ncy * H;
       } else if (t < kSlots + NY) {
         oy = t - kSlots;
         ox = ncx * H;
