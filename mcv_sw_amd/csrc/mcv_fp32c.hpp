@@ -183,21 +183,21 @@ __device__ __forceinline__ void stage_tile_f32(const MeshF32 &m, const StageArgs
   }
   __syncthreads();
 
+  // cell ends: a wavefront works along one direction (see stage_tile)
   constexpr int kTasksX = (CX + 1) * NY, kTasksY = (CY + 1) * NX;
-  for (int t = threadIdx.x; t < kTasksX + kTasksY; t += blockDim.x) {
-    const bool isx = t < kTasksX;
-    const int tt = isx ? t : t - kTasksX;
-    int mb, o;
-    if (isx) { mb = div_small<NY>(tt); o = tt - mb * NY; }
-    else { mb = div_small<NX>(tt); o = tt - mb * NX; }
-    if (isx ? (mb > ncx || o >= ny) : (mb > ncy || o >= nx)) continue;
-    const int st = isx ? 1 : TX;
+  constexpr int kStartY = (kTasksX + 63) / 64 * 64;
+  auto cell_end = [&](auto xdir, const int tt) {
+    constexpr bool isx = decltype(xdir)::value;
+    constexpr int nl = isx ? NY : NX;
+    const int mb = div_small<nl>(tt), o = tt - mb * nl;
+    if (isx ? (mb > ncx || o >= ny) : (mb > ncy || o >= nx)) return;
+    constexpr int st = isx ? 1 : TX;
     const int b = isx ? (o + H) * TX + (H + mb * H) : (H + mb * H) * TX + (o + H);
-    const C *sC = isx ? sCU : sCV;
-    const int cst = isx ? 1 : NX;  // the same line in the contravariant wind's slots
+    const C *const sC = isx ? sCU : sCV;
+    constexpr int cst = isx ? 1 : NX;  // the same line in the contravariant wind's slots
     const int cb = isx ? TL::cu_at(H + mb * H, o + H) : TL::cv_at(o + H, H + mb * H);
-    const C *sQ = isx ? sU : sV;
-    const C *sW = isx ? sV : sU;
+    const C *const sQ = isx ? sU : sV;
+    const C *const sW = isx ? sV : sU;
     const C c = sC[cb];
     // wave speed; phi to FP32 from phiG and the FP64 sqrtG
     const C phi =
@@ -240,11 +240,15 @@ __device__ __forceinline__ void stage_tile_f32(const MeshF32 &m, const StageArgs
       const C wlr = fit_right_t(wL, DOF, rdx, r2dx), wrl = fit_left_t(wR, DOF, rdx, r2dx);
       fW = riemann_t(wlr, wrl, wlr, wrl, up);
     }
-    if (isx) {
+    if constexpr (isx) {
       rxF[tt] = fF; rxD[tt] = fD; rxV[tt] = fW;
     } else {
       ryF[tt] = fF; ryD[tt] = fD; ryU[tt] = fW;
     }
+  };
+  for (int t = threadIdx.x; t < kStartY + kTasksY; t += blockDim.x) {
+    if (t < kTasksX) cell_end(std::true_type{}, t);
+    else if (t >= kStartY) cell_end(std::false_type{}, t - kStartY);
   }
   __syncthreads();
 

@@ -12,6 +12,8 @@
 // extents, so no index needs a run-time integer division.
 #pragma once
 
+#include <type_traits>
+
 #include "mcv_device.hpp"
 
 namespace mcv {
@@ -103,12 +105,12 @@ __device__ __forceinline__ void stage_tile(const MeshDev &m, const StageArgs &a,
 #pragma unroll
     for (int q = 0; q < kP0; ++q) {
       const int t = t0 + q * blockDim.x;
-      const int ly = t / TX, lx = t - ly * TX;
+      const int ly = div_small<TX>(t), lx = t - ly * TX;
       const bool inx = lx >= H && lx < H + nx, iny = ly >= H && ly < H + ny;
       // outside the tile, or a halo corner (never read)
       live[q] = t < TX * TY && lx < lw && ly < lh && (inx || iny);
       if (!live[q]) continue;
-      const uint32_t off = (uint32_t)((j0 - 1 + ly) * nh + (i0 - 1 + lx));
+      const uint32_t off = mul24(j0 - 1 + ly, nh) + (uint32_t)(i0 - 1 + lx);
       const uint32_t g = pbase + off;
       const D2 pu = ldg(a.in_pu, g);
       rphi[q] = pu.a;
@@ -129,7 +131,7 @@ __device__ __forceinline__ void stage_tile(const MeshDev &m, const StageArgs &a,
     for (int q = 0; q < kP0; ++q) {
       if (!live[q]) continue;
       const int li = t0 + q * blockDim.x;  // = ly * TX + lx
-      const int ly = li / TX, lx = li - ly * TX;
+      const int ly = div_small<TX>(li), lx = li - ly * TX;
       const double phi = rphi[q], u = ru[q], v = rv[q], g11 = r11[q], g12 = r12[q],
                    g22 = r22[q];
       double cu, cv;
@@ -154,29 +156,34 @@ __device__ __forceinline__ void stage_tile(const MeshDev &m, const StageArgs &a,
         // the wave speed's square root is left to phase 1, whose lanes are all
         // cell ends (one per thread there; here four, with most lanes idle:
         // MCV4 6x96^2 90.7 -> 88.9 us, 6x384^2 1078 -> 1070 us per RK4 step)
-        if (ox % H == 0) lamx[(ox / H) * NY + oy] = g11 * phi;
-        if (oy % H == 0) lamy[(oy / H) * NX + ox] = g22 * phi;
+        const int cx = div_small<H>(ox), cy = div_small<H>(oy);
+        if (ox == cx * H) lamx[cx * NY + oy] = g11 * phi;
+        if (oy == cy * H) lamy[cy * NX + ox] = g22 * phi;
       }
     }
   }
   __syncthreads();
 
-  // Phase 1: Riemann derivatives at every cell end of the core, x then y.
+  // Phase 1: Riemann derivatives at every cell end of the core, x then y.  The
+  // y tasks start on a wavefront of their own, so that a wavefront works along
+  // one direction and every LDS offset is a compile-time constant: 30 paired
+  // LDS reads for both directions where mixed lanes took 41 single ones with
+  // an address each (MCV4 6x384^2, per RK4 step: FP64 1030 -> 1001 us, FP32C
+  // 746 -> 724).
   constexpr int kTasksX = (CX + 1) * NY, kTasksY = (CY + 1) * NX;
-  for (int t = threadIdx.x; t < kTasksX + kTasksY; t += blockDim.x) {
-    const bool isx = t < kTasksX;
-    const int tt = isx ? t : t - kTasksX;
-    int mb, o;
-    if (isx) { mb = tt / NY; o = tt - mb * NY; }
-    else { mb = tt / NX; o = tt - mb * NX; }
-    if (isx ? (mb > ncx || o >= ny) : (mb > ncy || o >= nx)) continue;
-    const int st = isx ? 1 : TX;  // stride along the sweep
+  constexpr int kStartY = (kTasksX + 63) / 64 * 64;
+  auto cell_end = [&](auto xdir, const int tt) {
+    constexpr bool isx = decltype(xdir)::value;
+    constexpr int nl = isx ? NY : NX;  // lines across the sweep
+    const int mb = div_small<nl>(tt), o = tt - mb * nl;
+    if (isx ? (mb > ncx || o >= ny) : (mb > ncy || o >= nx)) return;
+    constexpr int st = isx ? 1 : TX;  // stride along the sweep
     const int b = isx ? (o + H) * TX + (H + mb * H) : (H + mb * H) * TX + (o + H);
-    const double *sC = isx ? sCU : sCV;
-    const int cst = isx ? 1 : NX;  // the same line in the contravariant wind's slots
+    const double *const sC = isx ? sCU : sCV;
+    constexpr int cst = isx ? 1 : NX;  // the same line in the contravariant wind's slots
     const int cb = isx ? TL::cu_at(H + mb * H, o + H) : TL::cv_at(o + H, H + mb * H);
-    const double *sQ = isx ? sU : sV;   // q of the gradient flux
-    const double *sW = isx ? sV : sU;   // upwinded cross wind
+    const double *const sQ = isx ? sU : sV;  // q of the gradient flux
+    const double *const sW = isx ? sV : sU;  // upwinded cross wind
     const double cb0 = sC[cb];
     const double lam = wave_speed(cb0, isx ? lamx[tt] : lamy[tt]);
     const double up = upwind_sign(cb0);
@@ -216,11 +223,15 @@ __device__ __forceinline__ void stage_tile(const MeshDev &m, const StageArgs &a,
       const double wlr = fit_right<DOF>(wL, dv), wrl = fit_left<DOF>(wR, dv);
       fW = riemann(wlr, wrl, wlr, wrl, up);
     }
-    if (isx) {
+    if constexpr (isx) {
       rxF[tt] = fF; rxD[tt] = fD; rxV[tt] = fW;
     } else {
       ryF[tt] = fF; ryD[tt] = fD; ryU[tt] = fW;
     }
+  };
+  for (int t = threadIdx.x; t < kStartY + kTasksY; t += blockDim.x) {
+    if (t < kTasksX) cell_end(std::true_type{}, t);
+    else if (t >= kStartY) cell_end(std::false_type{}, t - kStartY);
   }
   __syncthreads();
 
@@ -250,7 +261,7 @@ __device__ __forceinline__ void stage_tile(const MeshDev &m, const StageArgs &a,
       int ox = 0, oy = 0;
       bool ok = false;
       if (t < kSlots) {
-        oy = t / kRow;
+        oy = div_small<kRow>(t);
         ox = t - oy * kRow;
         ok = ox < ncx * H && oy < ncy * H;
       } else if (t < kSlots + NY) {
@@ -266,7 +277,7 @@ __device__ __forceinline__ void stage_tile(const MeshDev &m, const StageArgs &a,
       rox[q] = ox;
       roy[q] = oy;
       if (!ok) continue;
-      const uint32_t off = (uint32_t)((j0 + oy + H - 1) * nh + (i0 + ox + H - 1));
+      const uint32_t off = mul24(j0 + oy + H - 1, nh) + (uint32_t)(i0 + ox + H - 1);
       const uint32_t g = pbase + off;
       rf[q] = ldg(m.f, g);
       if (need_base) {
@@ -289,7 +300,7 @@ __device__ __forceinline__ void stage_tile(const MeshDev &m, const StageArgs &a,
       const int lx = ox + H, ly = oy + H, li = ly * TX + lx;
       double fx, dvx, vx, fy, dvy, uy;
       {  // x sweep
-        const int mb = ox / H, pos = ox - mb * H;
+        const int mb = div_small<H>(ox), pos = ox - mb * H;
         const int r0 = mb * NY + oy;
         if (pos == 0) {
           fx = rxF[r0]; dvx = rxD[r0]; vx = rxV[r0];
@@ -307,7 +318,7 @@ __device__ __forceinline__ void stage_tile(const MeshDev &m, const StageArgs &a,
         }
       }
       {  // y sweep
-        const int mb = oy / H, pos = oy - mb * H;
+        const int mb = div_small<H>(oy), pos = oy - mb * H;
         const int r0 = mb * NX + ox;
         if (pos == 0) {
           fy = ryF[r0]; dvy = ryD[r0]; uy = ryU[r0];
@@ -326,7 +337,7 @@ __device__ __forceinline__ void stage_tile(const MeshDev &m, const StageArgs &a,
         }
       }
       const int i = i0 + ox, j = j0 + oy;
-      const uint32_t g = pbase + (uint32_t)((j + H - 1) * nh + (i + H - 1));
+      const uint32_t g = pbase + mul24(j + H - 1, nh) + (uint32_t)(i + H - 1);
       const double sg = lds.sSG[TL::core_at(lx, ly)];
       const Recip sgr{sg, 1.0 / sg};  // the IEEE quotient, as the host forms RN(1/sqrtG)
       const double fc = rf[q];
