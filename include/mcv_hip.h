@@ -134,7 +134,8 @@ int mcv_hip_steps_done(const mcv_handle *h, int64_t *steps);
  * whole-program clock of MCV_SW.F90:33,80-82): like mcv_hip_step, but records
  * a HIP event after every kernel on the handle's stream, blocks, and returns
  * the summed durations of the stage kernels and of the boundary kernels in
- * milliseconds (either pointer may be NULL). */
+ * milliseconds (either pointer may be NULL).  Small solves run the boundary
+ * pass inside the stage kernels, with one boundary kernel at the end. */
 int mcv_hip_step_timed(mcv_handle *h, int32_t nsteps, double *stage_ms,
                        double *boundary_ms);
 

@@ -2,17 +2,22 @@
 //
 // A batch holds up to `capacity` solves (slots) of any order (MCV3/MCV4),
 // resolution, precision (FP64/FP32C), RK scheme (RK3_TVD/RK4) and time step.
-// Each stage (three launches) advances every listed solve by ONE RK stage:
+// Each stage launch advances every listed solve by ONE RK stage:
 //
 //   batch_stage_kernel     one workgroup per item of the concatenated
 //                          (solve, panel, tile) work list of all listed
 //                          solves, each at its own stage of its own scheme
 //                          (the stage index lives on the device, so solves
-//                          admitted at different times interleave freely)
+//                          admitted at different times interleave freely);
+//                          the first tile of a solve writes its advanced
+//                          progress to the other of two progress tables
 //   batch_boundary_kernel  one workgroup per unit of 256 boundary items of
 //                          every solve's freshly written level
-//   batch_advance_kernel   one workgroup; advances every solve's stage index
-//                          and step counters
+//
+// In a small batch the boundary kernel runs only after the last stage of a run:
+// between its stages batch_raw_stage_kernel takes the place of the stage
+// kernel, whose tiles at the panel sides run the pass on the points they stage.
+// After a run every level is finished, as the read-backs expect it.
 //
 // All per-solve data the kernels need sits in device tables (solve
 // descriptors, stage state, work prefix sums), so one captured hipGraph of
@@ -52,16 +57,35 @@ struct BatchSolve {
   StageArgs32 a32[kMaxStages];
   BoundaryArgs b64[kMaxStages];
   BoundaryArgs32 b32[kMaxStages];
-  const double *cu0, *cv0;  // handed-over contravariant winds (FP64, first stage)
 };
 
-// Mutable progress of one solve, advanced on the device.
+// Mutable progress of one solve, advanced on the device.  A stage launch reads
+// one table and writes the advanced entries to the other, so that no workgroup
+// sees an entry change under it.
 struct BatchProgress {
   int phase;           // next stage index
   int first;           // no stage has run yet
   long long steps_left;
   long long steps_done;
 };
+
+// Stages a solve has run: the boundary kernel stamps the solves it finishes
+// with this number, and a stage whose input bears it reads a finished level.
+__device__ __forceinline__ long long stages_run(const BatchProgress &st, int nstages) {
+  return st.steps_done * nstages + st.phase;
+}
+
+// The progress after one more stage (a spent solve stays as it is).
+__device__ __forceinline__ BatchProgress advanced(BatchProgress st, int nstages) {
+  if (st.steps_left <= 0) return st;
+  st.first = 0;
+  if (++st.phase == nstages) {
+    st.phase = 0;
+    --st.steps_left;
+    ++st.steps_done;
+  }
+  return st;
+}
 
 // Bodies of the batched stage kernel: (precision, order) pairs, and the RK
 // schemes its solves use.  A kernel instantiation compiles the bodies of its
@@ -150,9 +174,11 @@ __device__ __forceinline__ int find_entry(const int *prefix, int cnt, int w) {
 // least 8 * ceil(items / 8) workgroups, so each takes at most one item and the
 // hardware's dynamic dispatch balances the tiles; a smaller grid would walk
 // the chunk in strides.
-template <int V, int M>
+// Raw: a solve's input may be as a stage left it (its stamp tells).
+template <int V, int M, bool Raw>
 __device__ __forceinline__ void batch_stage_items(
     const BatchSolve *__restrict__ solves, const BatchProgress *__restrict__ prog,
+    BatchProgress *__restrict__ next, const long long *__restrict__ stamp,
     const int *__restrict__ list, const int *__restrict__ wprefix, const int *__restrict__ meta,
     char *smem) {
   const int cnt = meta[0];
@@ -171,9 +197,11 @@ __device__ __forceinline__ void batch_stage_items(
     }
     const int sl = list[k];
     const BatchProgress st = prog[sl];
-    if (st.steps_left <= 0) continue;
     const BatchSolve &S = solves[sl];
     const int local = w - wprefix[k];
+    if (local == 0 && threadIdx.x == 0) next[sl] = advanced(st, S.nstages);
+    if (st.steps_left <= 0) continue;
+    const bool raw = Raw && stamp[sl] != stages_run(st, S.nstages);
     const int p = local % 6 + 1, tile = local / 6;
     const int ph = st.phase, kind = S.kind[ph];
     // the host launches a mask holding the scheme of every solve in the batch
@@ -183,19 +211,21 @@ __device__ __forceinline__ void batch_stage_items(
     // the host launches a mask holding every body in the batch
     if (S.prec == MCV_FP64) {
       if constexpr ((M & (kBody64x3 | kBody64x4)) != 0) {
-        StageArgs a = S.a64[ph];
-        if (st.first) { a.cu0 = S.cu0; a.cv0 = S.cv0; }
-        const MeshDev &m = S.mesh;  // read where used (scalar loads), not copied
+        const StageArgs &a = S.a64[ph];  // read where used (scalar loads), not copied
+        const MeshDev &m = S.mesh;
+        const bool winds = st.first != 0;
         if (S.dof == 3) {
           if constexpr ((M & kBody64x3) != 0) {
             const int tx = tiles_x_of<V>(3, MCV_FP64, n);
-            stage_tile<3, TileSet<3>::cx[V], TileSet<3>::cy[V]>(m, a, kind, p, tile % tx,
+            stage_tile<3, TileSet<3>::cx[V], TileSet<3>::cy[V], false>(m, a, kind, raw, winds, p,
+                                                                 tile % tx,
                                                                  tile / tx, smem);
           }
         } else {
           if constexpr ((M & kBody64x4) != 0) {
             const int tx = tiles_x_of<V>(4, MCV_FP64, n);
-            stage_tile<4, TileSet<4>::cx[V], TileSet<4>::cy[V]>(m, a, kind, p, tile % tx,
+            stage_tile<4, TileSet<4>::cx[V], TileSet<4>::cy[V], false>(m, a, kind, raw, winds, p,
+                                                                 tile % tx,
                                                                  tile / tx, smem);
           }
         }
@@ -207,13 +237,13 @@ __device__ __forceinline__ void batch_stage_items(
         if (S.dof == 3) {
           if constexpr ((M & kBody32x3) != 0) {
             const int tx = tiles_x_of<V>(3, MCV_FP32C, n);
-            stage_tile_f32<3, TileSet32<3>::cx[V], TileSet32<3>::cy[V]>(m, a, kind, p, tile % tx,
+            stage_tile_f32<3, TileSet32<3>::cx[V], TileSet32<3>::cy[V], false>(m, a, kind, raw, p, tile % tx,
                                                                         tile / tx, smem);
           }
         } else {
           if constexpr ((M & kBody32x4) != 0) {
             const int tx = tiles_x_of<V>(4, MCV_FP32C, n);
-            stage_tile_f32<4, TileSet32<4>::cx[V], TileSet32<4>::cy[V]>(m, a, kind, p, tile % tx,
+            stage_tile_f32<4, TileSet32<4>::cx[V], TileSet32<4>::cy[V], false>(m, a, kind, raw, p, tile % tx,
                                                                         tile / tx, smem);
           }
         }
@@ -234,28 +264,64 @@ constexpr bool eight_waves(int V, int M) {
   return V == 0 || (V == 2 && bodies == kBody32x3);
 }
 
+// Waves per SIMD of the raw builds (the boundary pass would take registers
+// freely, see stage_waves): eight_waves' choice, else those of the bodies' single-solve kernels,
+// one less where a kernel holds several bodies (whose tables take registers too).
+template <int V>
+constexpr int batch_waves_v(int M) {
+  int w = 8;
+  auto take = [&](int body, int waves) { if ((M & body) && waves < w) w = waves; };
+  take(kBody64x3, stage_waves<double, 3, TileSet<3>::cx[V], TileSet<3>::cy[V]>());
+  take(kBody64x4, stage_waves<double, 4, TileSet<4>::cx[V], TileSet<4>::cy[V]>());
+  take(kBody32x3, stage_waves<FP32CStencil, 3, TileSet32<3>::cx[V], TileSet32<3>::cy[V]>());
+  take(kBody32x4, stage_waves<FP32CStencil, 4, TileSet32<4>::cx[V], TileSet32<4>::cy[V]>());
+  const int bodies = M & (kBody64x3 | kBody64x4 | kBody32x3 | kBody32x4);
+  if ((bodies & (bodies - 1)) != 0 && w > 4) --w;
+  if ((M & kBody64x4) != 0 && w > 5) w = 5;
+  return w < 6 ? w : 6;
+}
+constexpr int batch_waves(int V, int M) {
+  return eight_waves(V, M) ? 8 : V == 0 ? batch_waves_v<0>(M) : V == 1 ? batch_waves_v<1>(M)
+       : V == 2 ? batch_waves_v<2>(M) : batch_waves_v<3>(M);
+}
+
 template <int V, int M>
 __global__ __launch_bounds__(kStageThreads) void batch_stage_kernel(
     const BatchSolve *__restrict__ solves, const BatchProgress *__restrict__ prog,
-    const int *__restrict__ list, const int *__restrict__ wprefix, const int *__restrict__ meta) {
+    BatchProgress *__restrict__ next, const int *__restrict__ list,
+    const int *__restrict__ wprefix, const int *__restrict__ meta) {
   __shared__ __align__(16) char smem[BatchSmem<V, M>::kBytes];
-  batch_stage_items<V, M>(solves, prog, list, wprefix, meta, smem);
+  batch_stage_items<V, M, false>(solves, prog, next, nullptr, list, wprefix, meta, smem);
 }
 
 template <int V, int M>
 __global__ __launch_bounds__(kStageThreads) __attribute__((amdgpu_waves_per_eu(8, 8))) void
 batch_stage_kernel_8w(const BatchSolve *__restrict__ solves, const BatchProgress *__restrict__ prog,
-                      const int *__restrict__ list, const int *__restrict__ wprefix,
-                      const int *__restrict__ meta) {
+                      BatchProgress *__restrict__ next, const int *__restrict__ list,
+                      const int *__restrict__ wprefix, const int *__restrict__ meta) {
   __shared__ __align__(16) char smem[BatchSmem<V, M>::kBytes];
-  batch_stage_items<V, M>(solves, prog, list, wprefix, meta, smem);
+  batch_stage_items<V, M, false>(solves, prog, next, nullptr, list, wprefix, meta, smem);
 }
 
-// Boundary kernel: the boundary pass of every listed solve's freshly written
-// level, in work units of kBndChunk items.  The host launches at least one
-// workgroup per unit; a smaller grid would walk the units in strides.
-__global__ __launch_bounds__(256) void batch_boundary_kernel(
+template <int V, int M>
+__global__ __launch_bounds__(kStageThreads, batch_waves(V, M)) void batch_raw_stage_kernel(
     const BatchSolve *__restrict__ solves, const BatchProgress *__restrict__ prog,
+    BatchProgress *__restrict__ next, const long long *__restrict__ stamp,
+    const int *__restrict__ list, const int *__restrict__ wprefix, const int *__restrict__ meta) {
+  __shared__ __align__(16) char smem[BatchSmem<V, M>::kBytes];
+  batch_stage_items<V, M, true>(solves, prog, next, stamp, list, wprefix, meta, smem);
+}
+
+// Boundary kernel: the boundary pass of every listed solve's last written
+// level, in work units of kBndChunk items, and the stamp that says so.  `prev`:
+// the progress before the stage, after each of which the pass runs (spent
+// solves are passed over); null at the end of a run of raw stages (a level
+// finished before comes out the same, as the pass reads the band only).  The
+// host launches at least one workgroup per unit; a smaller grid would walk the
+// units in strides.
+__global__ __launch_bounds__(256) void batch_boundary_kernel(
+    const BatchSolve *__restrict__ solves, const BatchProgress *__restrict__ prev,
+    const BatchProgress *__restrict__ prog, long long *__restrict__ stamp,
     const int *__restrict__ list, const int *__restrict__ bprefix, const int *__restrict__ meta) {
   const int cnt = meta[0];
   const int total = cnt ? bprefix[cnt] : 0;
@@ -266,17 +332,19 @@ __global__ __launch_bounds__(256) void batch_boundary_kernel(
       kend = bprefix[k + 1];
     }
     const int sl = list[k];
+    if (prev && prev[sl].steps_left <= 0) continue;
     const BatchProgress st = prog[sl];
-    if (st.steps_left <= 0) continue;
     const BatchSolve &S = solves[sl];
-    const int ph = st.phase;
     const int base = (w - bprefix[k]) * kBndChunk;
+    if (base == 0 && threadIdx.x == 0) stamp[sl] = stages_run(st, S.nstages);
+    if (stages_run(st, S.nstages) == 0) continue;  // still the handed-over state
+    const int ph = (st.phase == 0 ? S.nstages : st.phase) - 1;  // the stage that wrote it
     const int lim = min(kBndChunk, S.nbitems - base);
     if (S.prec == MCV_FP64) {
       const BoundaryArgs b = S.b64[ph];
       for (int j = threadIdx.x; j < lim; j += blockDim.x) {
-        if (S.dof == 3) boundary_item<3>(S.mesh, b, base + j);
-        else boundary_item<4>(S.mesh, b, base + j);
+        if (S.dof == 3) boundary_item_f64<3>(S.mesh, b, base + j);
+        else boundary_item_f64<4>(S.mesh, b, base + j);
       }
     } else {
       const BoundaryArgs32 b = S.b32[ph];
@@ -285,27 +353,6 @@ __global__ __launch_bounds__(256) void batch_boundary_kernel(
         else boundary_item_f32<4>(S.mesh, b, base + j);
       }
     }
-  }
-}
-
-// Advances every listed solve by one stage (stage index, then step counters);
-// one workgroup, after the boundary kernel of the stage.
-__global__ __launch_bounds__(256) void batch_advance_kernel(const BatchSolve *__restrict__ solves,
-                                                            BatchProgress *__restrict__ prog,
-                                                            const int *__restrict__ list,
-                                                            const int *__restrict__ meta) {
-  const int cnt = meta[0];
-  for (int e = threadIdx.x; e < cnt; e += blockDim.x) {
-    const int sl = list[e];
-    BatchProgress st = prog[sl];
-    if (st.steps_left <= 0) continue;
-    st.first = 0;
-    if (++st.phase == solves[sl].nstages) {
-      st.phase = 0;
-      --st.steps_left;
-      ++st.steps_done;
-    }
-    prog[sl] = st;
   }
 }
 
@@ -321,7 +368,11 @@ struct mcv_batch {
   std::vector<BatchSolve> solve;        // host copies of the descriptors
   std::vector<BatchProgress> progress;  // host view, refreshed by poll
   BatchSolve *d_solve = nullptr;
+  // progress: two tables of `capacity` entries; table 0 is current between runs,
+  // table `cur` within one
   BatchProgress *d_prog = nullptr;
+  int cur = 0;
+  long long *d_stamp = nullptr;  // stages run when the boundary kernel last finished a solve
   int *d_list = nullptr, *d_wprefix = nullptr, *d_bprefix = nullptr, *d_meta = nullptr;
   std::vector<void *> allocs;
   int variant = 0;
@@ -330,10 +381,12 @@ struct mcv_batch {
   int stage_grid = 0;   // workgroups of the stage launch (>= 8 * ceil(items / 8))
   int bnd_units = 0;    // boundary work units
   int bnd_grid = 0;     // workgroups of the boundary launch (>= units)
+  bool fused = false;   // the boundary pass runs inside the stages (sides_in_stage)
   int mask = kNumMasks - 1;  // index into kBodyMasks of the launched stage kernel
   bool use_graph = true;
   hipGraphExec_t exec = nullptr;
   int exec_variant = -1, exec_mask = -1, exec_grid = 0, exec_bnd_grid = 0;
+  bool exec_fused = false;
   hipEvent_t ev[3] = {};
   int64_t stages_run = 0;
 };
@@ -381,27 +434,19 @@ BatchSolve describe(const mcv_handle *h) {
   s.nbitems = boundary_items(h->cfg.dof, h->npv);
   s.mesh = h->mesh;
   s.mesh32 = h->mesh32;
-  const double dt = h->cfg.dt;
-  struct St { int kind, in, out; double c1; };
-  // time_scheme_mod.F90:13-69 with the level roles of the single-solve path
-  const St rk4[4] = {{kRK4S1, 0, 1, 0.5 * dt}, {kRK4S2, 1, 2, 0.5 * dt}, {kRK4S3, 2, 1, dt},
-                     {kRK4S4, 1, 0, dt}};
-  const St rk3[3] = {{kRK3S1, 0, 1, dt}, {kRK3S2, 1, 2, 0.25 * dt},
-                     {kRK3S3, 2, 0, 2.0 / 3.0 * dt}};
-  const St *sched = h->cfg.scheme == MCV_RK4 ? rk4 : rk3;
-  s.nstages = h->cfg.scheme == MCV_RK4 ? 4 : 3;
+  s.nstages = stage_count(h->cfg.scheme);
   for (int i = 0; i < s.nstages; ++i) {
-    s.kind[i] = sched[i].kind;
+    s.kind[i] = stage_spec(h->cfg, i).kind;
     if (h->fp32c) {
-      s.a32[i] = stage_args32(h, sched[i].in, sched[i].out, sched[i].c1);
-      s.b32[i] = boundary_args32(h, sched[i].out);
+      s.a32[i] = stage_args32(h, i);
+      s.b32[i] = boundary_args32(h, i);
     } else {
-      s.a64[i] = stage_args64(h, sched[i].in, sched[i].out, sched[i].c1);
-      s.b64[i] = boundary_args64(h, sched[i].out);
+      s.a64[i] = stage_args64(h, i);
+      s.b64[i] = boundary_args64(h, i);
     }
   }
-  s.cu0 = h->cu0;
-  s.cv0 = h->cv0;
+  s.a64[0].cu0 = h->cu0;  // read by the solve's first stage
+  s.a64[0].cv0 = h->cv0;
   return s;
 }
 
@@ -445,6 +490,7 @@ int upload_tables(mcv_batch *b) {
   // the host vectors go out of scope: finish the copies first
   HIP_TRY(hipStreamSynchronize(b->stream));
   b->mask = mask_index(need);
+  b->fused = sides_in_stage(b->variant, b->stage_items);
   // a graph keeps its grids while the work fits in them and fills at least
   // half of them
   auto keep = [&](int have, int fit) {
@@ -458,13 +504,23 @@ int upload_tables(mcv_batch *b) {
 
 template <int V, int I>
 void launch_stage_vm(mcv_batch *b) {
+  BatchProgress *const prog = b->d_prog + b->cur * b->capacity;
+  BatchProgress *const next = b->d_prog + (1 - b->cur) * b->capacity;
+  if constexpr (V == 0 || V == 2) {
+    if (b->fused) {
+      hipLaunchKernelGGL((batch_raw_stage_kernel<V, kBodyMasks[I]>), dim3(b->stage_grid),
+                         dim3(kStageThreads), 0, b->stream, b->d_solve, prog, next, b->d_stamp,
+                         b->d_list, b->d_wprefix, b->d_meta);
+      return;
+    }
+  }
   if constexpr (eight_waves(V, kBodyMasks[I])) {
     hipLaunchKernelGGL((batch_stage_kernel_8w<V, kBodyMasks[I]>), dim3(b->stage_grid),
-                       dim3(kStageThreads), 0, b->stream, b->d_solve, b->d_prog, b->d_list,
+                       dim3(kStageThreads), 0, b->stream, b->d_solve, prog, next, b->d_list,
                        b->d_wprefix, b->d_meta);
   } else {
     hipLaunchKernelGGL((batch_stage_kernel<V, kBodyMasks[I]>), dim3(b->stage_grid),
-                       dim3(kStageThreads), 0, b->stream, b->d_solve, b->d_prog, b->d_list,
+                       dim3(kStageThreads), 0, b->stream, b->d_solve, prog, next, b->d_list,
                        b->d_wprefix, b->d_meta);
   }
 }
@@ -492,28 +548,45 @@ int launch_stage(mcv_batch *b, int v) {
   return MCV_OK;
 }
 
-int launch_boundary(mcv_batch *b) {
+// The boundary pass on every listed solve's last level; after one stage, or (a
+// run of raw stages) after the last.
+int launch_boundary(mcv_batch *b, bool after_one) {
+  BatchProgress *const prog = b->d_prog + b->cur * b->capacity;
+  BatchProgress *const prev = after_one ? b->d_prog + (1 - b->cur) * b->capacity : nullptr;
   hipLaunchKernelGGL(batch_boundary_kernel, dim3(b->bnd_grid), dim3(256), 0, b->stream,
-                     b->d_solve, b->d_prog, b->d_list, b->d_bprefix, b->d_meta);
-  HIP_TRY(hipGetLastError());
-  hipLaunchKernelGGL(batch_advance_kernel, dim3(1), dim3(256), 0, b->stream, b->d_solve,
-                     b->d_prog, b->d_list, b->d_meta);
+                     b->d_solve, prev, prog, b->d_stamp, b->d_list, b->d_bprefix, b->d_meta);
   HIP_TRY(hipGetLastError());
   return MCV_OK;
 }
 
-int launch_pair(mcv_batch *b) {
-  int rc = launch_stage(b, b->variant);
-  return rc ? rc : launch_boundary(b);
+// One stage of every listed solve.
+int run_stage(mcv_batch *b) {
+  const int rc = launch_stage(b, b->variant);
+  if (rc) return rc;
+  b->cur = 1 - b->cur;
+  return b->fused ? MCV_OK : launch_boundary(b, true);
+}
+
+// The end of a run: every level finished, progress table 0 current.
+int finish_run(mcv_batch *b) {
+  int rc;
+  if (b->fused && (rc = launch_boundary(b, false))) return rc;
+  if (b->cur) {
+    HIP_TRY(hipMemcpyAsync(b->d_prog, b->d_prog + b->capacity, sizeof(BatchProgress) * b->capacity,
+                           hipMemcpyDeviceToDevice, b->stream));
+    b->cur = 0;
+  }
+  return MCV_OK;
 }
 
 int capture(mcv_batch *b) {
   drop_graph(b);
   HIP_TRY(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
   int rc = MCV_OK;
-  for (int i = 0; i < kGraphStages && rc == MCV_OK; ++i) rc = launch_pair(b);
+  for (int i = 0; i < kGraphStages && rc == MCV_OK; ++i) rc = run_stage(b);
   hipGraph_t g = nullptr;
   const hipError_t e = hipStreamEndCapture(b->stream, &g);
+  b->cur = 0;  // nothing has run yet
   if (rc) {
     if (g) (void)hipGraphDestroy(g);
     return rc;
@@ -530,6 +603,7 @@ int capture(mcv_batch *b) {
   b->exec_mask = b->mask;
   b->exec_grid = b->stage_grid;
   b->exec_bnd_grid = b->bnd_grid;
+  b->exec_fused = b->fused;
   return MCV_OK;
 }
 
@@ -575,8 +649,10 @@ int mcv_batch_create(int32_t device, int32_t capacity, mcv_batch **out) {
     HIP_TRY(hipStreamCreate(&b->stream));
     for (hipEvent_t &e : b->ev) HIP_TRY(hipEventCreate(&e));
     int rc;
-    if ((rc = balloc(b, &b->d_solve, capacity)) || (rc = balloc(b, &b->d_prog, capacity)) ||
-        (rc = balloc(b, &b->d_list, capacity)) || (rc = balloc(b, &b->d_wprefix, capacity + 1)) ||
+    if ((rc = balloc(b, &b->d_solve, capacity)) ||
+        (rc = balloc(b, &b->d_prog, 2 * (size_t)capacity)) ||
+        (rc = balloc(b, &b->d_stamp, capacity)) || (rc = balloc(b, &b->d_list, capacity)) ||
+        (rc = balloc(b, &b->d_wprefix, capacity + 1)) ||
         (rc = balloc(b, &b->d_bprefix, capacity + 1)) || (rc = balloc(b, &b->d_meta, 4)))
       return rc;
     HIP_TRY(hipMemcpy(b->d_prog, b->progress.data(), sizeof(BatchProgress) * capacity,
@@ -619,6 +695,9 @@ int mcv_batch_add(mcv_batch *b, const mcv_config *cfg, const mcv_mesh *mesh,
                          b->stream));
   HIP_TRY(hipMemcpyAsync(b->d_prog + s, &b->progress[s], sizeof(BatchProgress),
                          hipMemcpyHostToDevice, b->stream));
+  const long long stages = 0;
+  HIP_TRY(hipMemcpyAsync(b->d_stamp + s, &stages, sizeof(stages), hipMemcpyHostToDevice,
+                         b->stream));
   HIP_TRY(hipStreamSynchronize(b->stream));
   b->slot[s] = h;
   b->tables_dirty = true;
@@ -647,14 +726,16 @@ int mcv_batch_run(mcv_batch *b, int32_t nstages) {
   int left = nstages;
   if (b->use_graph && left >= kGraphStages) {
     if (!b->exec || b->exec_variant != b->variant || b->exec_mask != b->mask ||
-        b->exec_grid != b->stage_grid || b->exec_bnd_grid != b->bnd_grid) {
+        b->exec_grid != b->stage_grid || b->exec_bnd_grid != b->bnd_grid ||
+        b->exec_fused != b->fused) {
       if ((rc = capture(b))) return rc;
     }
     for (; left >= kGraphStages; left -= kGraphStages)
       HIP_TRY(hipGraphLaunch(b->exec, b->stream));
   }
   for (; left > 0; --left)
-    if ((rc = launch_pair(b))) return rc;
+    if ((rc = run_stage(b))) return rc;
+  if (nstages > 0 && (rc = finish_run(b))) return rc;
   b->stages_run += nstages;
   return MCV_OK;
 }
@@ -751,18 +832,26 @@ int mcv_batch_run_timed(mcv_batch *b, int32_t nstages, double *stage_ms, double 
   int rc;
   if (b->tables_dirty && (rc = upload_tables(b))) return rc;
   double sm = 0.0, bm = 0.0;
+  // the boundary pass after each stage, or after the last one
   for (int i = 0; i < nstages; ++i) {
+    const bool pass = !b->fused || i == nstages - 1;
     HIP_TRY(hipEventRecord(b->ev[0], b->stream));
     if ((rc = launch_stage(b, b->variant))) return rc;
+    b->cur = 1 - b->cur;
     HIP_TRY(hipEventRecord(b->ev[1], b->stream));
-    if ((rc = launch_boundary(b))) return rc;
+    if (pass && (rc = launch_boundary(b, !b->fused))) return rc;
     HIP_TRY(hipEventRecord(b->ev[2], b->stream));
     HIP_TRY(hipEventSynchronize(b->ev[2]));
     float a = 0.f, c = 0.f;
     HIP_TRY(hipEventElapsedTime(&a, b->ev[0], b->ev[1]));
     HIP_TRY(hipEventElapsedTime(&c, b->ev[1], b->ev[2]));
     sm += a;
-    bm += c;
+    if (pass) bm += c;
+  }
+  if (nstages > 0 && b->cur) {
+    HIP_TRY(hipMemcpyAsync(b->d_prog, b->d_prog + b->capacity, sizeof(BatchProgress) * b->capacity,
+                           hipMemcpyDeviceToDevice, b->stream));
+    b->cur = 0;
   }
   b->stages_run += nstages;
   if (stage_ms) *stage_ms = sm;

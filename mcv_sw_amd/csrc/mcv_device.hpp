@@ -10,6 +10,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 namespace mcv {
 
 // ---------------------------------------------------------------------------
@@ -63,6 +65,10 @@ struct alignas(8) F2 {
 struct alignas(4) F3 {
   float a, b, c;
 };
+// Three doubles as one 24-byte record (a 16-byte and an 8-byte access).
+struct alignas(8) D3 {
+  double a, b, c;
+};
 // Four floats loaded together (one 16-byte load).
 struct alignas(16) F4 {
   float a, b, c, d;
@@ -72,21 +78,19 @@ struct MeshDev {
   int dof, n, npv, nh;
   double dx;                 // element width, radians
   MCVDivisors dv;            // dx, 2dx, dx^2 with their reciprocals
-  long long metric_pstride;  // panel stride of sqrtG, rsqrtG, ig11, ig12, ig22
+  long long metric_pstride;  // panel stride of sqrtG, ig11, ig12, ig22, mpack
   long long phis_pstride;    // panel stride of phi_s
-  const double *sqrtG, *rsqrtG, *ig11, *ig12, *ig22;  // rsqrtG = RN(1/sqrtG)
+  const double *sqrtG, *ig11, *ig12, *ig22;
   // The same metric terms packed per point for the stage kernel, so that a
-  // point's terms come in one or two 16-byte loads (metric_pstride applies):
+  // point's terms come in two 16-byte loads:
   const D2 *mpack;  // 2 per point: {sqrtG, IG11}, {IG12, IG22}
-  const D2 *spack;  // 1 per point: {sqrtG, 1/sqrtG}
   int phis_zero;    // phi_s is +0.0 at every point (not read; adding +0.0 is exact)
   const double *f;           // per panel (f differs between panels 5 and 6)
   const double *phi_s;
   const double *p2sp;        // (A*IG) per point, 4 doubles (m11, m21, m12, m22)
   // Line-major copies for the boundary pass (4 doubles per point):
-  const double *p2sp_band;   // (A*IG) on the band lines, see band_point()
   const double *sp2p_ghost;  // (G*IA) at the ghost points, see ghost_point()
-  const double *sp2p_edge;   // (G*IA) on the edge lines, see band_point() with d = 1
+  const double *sp2p_edge;   // (G*IA) on the edge lines, see edge_point()
   const double *gcoef;       // (H, nPV): ghost offsets (ghost_mod.f90:11-18)
   const int32_t *giref;      // (H, nPV): 1-based cells
 };
@@ -103,7 +107,10 @@ struct StageArgs {
   double *acc_v;                       //   and v
   D2 *o_pu;                            // stage output (interior, raw); the tendency seam
   double *o_v;                         //   writes {phiG, u} and v tendencies on (nPV, nPV, 6)
-  double *band_raw;                    // raw copy of the lines nearest each side, see band_slot()
+  D3 *band_raw;                        // raw copy of the lines nearest each side, see band_point()
+  const D3 *band_in;                   // the band of the stage that wrote in_pu, in_v
+  D2 *fin_pu;                          // level whose edge lines a raw input's owners finish
+  double *fin_v;                       //   (Y_n, a later stage's base), or null
   const double *cu0, *cv0;             // host contravariant winds (first stage only)
   double c1;                           // stage increment coefficient (x dt)
 };
@@ -111,7 +118,7 @@ struct StageArgs {
 struct BoundaryArgs {
   D2 *pu;                              // level to finish (halo + edges)
   double *v;
-  const double *band_raw;
+  const D3 *band_raw;
 };
 
 // Stage kinds of time_scheme_mod.F90:13-123.
@@ -129,17 +136,11 @@ enum StageKind : int {
 // The band: the H+1 lines nearest each side (0 W, 1 E, 2 S, 3 N) of each
 // panel p (1..6), as the stage kernel wrote them (before the boundary pass).
 // Depth d = 1 is the edge line; the along-line index al (1..nPV) is j on the
-// W/E sides and i on the S/N sides.  The boundary pass reads only the band,
-// contiguously along the lines.
+// W/E sides and i on the S/N sides.  One {phi, zonal, meridional} record per
+// point.  The boundary pass reads only the band, contiguously along the lines.
 __host__ __device__ inline uint32_t band_point(int npv, int H, int p, int side, int d, int al) {
   return (((uint32_t)(p - 1) * 4u + (uint32_t)side) * (uint32_t)(H + 1) + (uint32_t)(d - 1)) *
              (uint32_t)npv + (uint32_t)(al - 1);
-}
-// field 0 phi, 1 u, 2 v
-__host__ __device__ inline uint32_t band_slot(int npv, int H, int p, int side, int d, int field,
-                                              int al) {
-  return ((((uint32_t)(p - 1) * 4u + (uint32_t)side) * (uint32_t)(H + 1) + (uint32_t)(d - 1)) * 3u +
-          (uint32_t)field) * (uint32_t)npv + (uint32_t)(al - 1);
 }
 // Ghost point at depth k (1..H) beyond side `side` of panel p, along index s.
 __host__ __device__ inline uint32_t ghost_point(int npv, int H, int p, int side, int k, int s) {
@@ -157,9 +158,9 @@ __host__ __device__ inline void band_ij(int npv, int side, int d, int al, int &i
 __host__ __device__ inline uint32_t edge_point(int npv, int p, int side, int al) {
   return ((uint32_t)(p - 1) * 4u + (uint32_t)side) * (uint32_t)npv + (uint32_t)(al - 1);
 }
-// Band lines per solve (all panels, sides, depths and fields).
-__host__ __device__ inline size_t band_values(int dof, int npv) {
-  return (size_t)6 * 4 * dof * 3 * npv;
+// Band points per solve (all panels, sides and depths).
+__host__ __device__ inline size_t band_points(int dof, int npv) {
+  return (size_t)6 * 4 * dof * npv;
 }
 
 // Work items of the boundary pass on one level: every ghost point (6 panels
@@ -202,25 +203,72 @@ __device__ __forceinline__ int div_small(int t) {
 // byte offset, which the global load/store instructions take directly (no
 // 64-bit address arithmetic per access).  The library keeps every array that
 // the stage kernels touch below 2^32 bytes (n <= 2048).
+// The accesses name the global address space: a pointer that comes out of a
+// struct in memory is generic to the compiler, and a generic (flat) access
+// counts as an LDS access as well, so that every LDS wait would wait for it.
+#if defined(__HIP_DEVICE_COMPILE__)
+#define MCV_GLOBAL __attribute__((address_space(1)))
+#else
+#define MCV_GLOBAL
+#endif
+typedef double mcv_d2 __attribute__((__vector_size__(16)));
+typedef float mcv_f4 __attribute__((__vector_size__(16)));
+
+template <typename S>
+__device__ __forceinline__ S read_as(const MCV_GLOBAL char *p) {
+  return *(const MCV_GLOBAL S *)p;
+}
+template <typename S>
+__device__ __forceinline__ void write_as(MCV_GLOBAL char *p, S v) {
+  *(MCV_GLOBAL S *)p = v;
+}
+template <typename T>
+__device__ __forceinline__ T read_global(const MCV_GLOBAL char *p) {
+  if constexpr (std::is_same_v<T, D2>) {
+    const mcv_d2 v = read_as<mcv_d2>(p);
+    return D2{v[0], v[1]};
+  } else if constexpr (std::is_same_v<T, F4>) {
+    const mcv_f4 v = read_as<mcv_f4>(p);
+    return F4{v[0], v[1], v[2], v[3]};
+  } else if constexpr (std::is_same_v<T, D3>) {
+    return D3{read_as<double>(p), read_as<double>(p + 8), read_as<double>(p + 16)};
+  } else if constexpr (std::is_same_v<T, F3>) {
+    return F3{read_as<float>(p), read_as<float>(p + 4), read_as<float>(p + 8)};
+  } else {
+    return read_as<T>(p);
+  }
+}
+template <typename T>
+__device__ __forceinline__ void write_global(MCV_GLOBAL char *p, const T &v) {
+  if constexpr (std::is_same_v<T, D2>) {
+    write_as(p, mcv_d2{v.a, v.b});
+  } else if constexpr (std::is_same_v<T, D3>) {
+    write_as(p, v.a); write_as(p + 8, v.b); write_as(p + 16, v.c);
+  } else if constexpr (std::is_same_v<T, F3>) {
+    write_as(p, v.a); write_as(p + 4, v.b); write_as(p + 8, v.c);
+  } else {
+    write_as(p, v);
+  }
+}
+
 template <typename T>
 __device__ __forceinline__ T ldg(const T *base, uint32_t idx) {
-  return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(base) +
-                                      (size_t)(idx * (uint32_t)sizeof(T)));
+  return read_global<T>((const MCV_GLOBAL char *)base + (size_t)(idx * (uint32_t)sizeof(T)));
 }
 template <typename T>
 __device__ __forceinline__ void stg(T *base, uint32_t idx, T v) {
-  *reinterpret_cast<T *>(reinterpret_cast<char *>(base) + (size_t)(idx * (uint32_t)sizeof(T))) = v;
+  write_global((MCV_GLOBAL char *)base + (size_t)(idx * (uint32_t)sizeof(T)), v);
 }
 
 // The same at a byte offset formed by the caller (for 12-byte records, whose
 // offset idx * 12 would otherwise take a quarter-rate multiply).
 template <typename T>
 __device__ __forceinline__ T ldgb(const T *base, uint32_t byte_off) {
-  return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(base) + (size_t)byte_off);
+  return read_global<T>((const MCV_GLOBAL char *)base + (size_t)byte_off);
 }
 template <typename T>
 __device__ __forceinline__ void stgb(T *base, uint32_t byte_off, T v) {
-  *reinterpret_cast<T *>(reinterpret_cast<char *>(base) + (size_t)byte_off) = v;
+  write_global((MCV_GLOBAL char *)base + (size_t)byte_off, v);
 }
 
 // Linear index of point (i, j) of panel p (1-based, halo-relative i, j).
@@ -263,6 +311,9 @@ static __constant__ VtxPt kVerts[8][3] = {
     {{3, 0, 1}, {2, 1, 1}, {5, 1, 1}}, {{3, 1, 1}, {4, 0, 1}, {5, 0, 1}},
     {{2, 1, 0}, {3, 0, 0}, {6, 1, 0}}, {{3, 1, 0}, {4, 0, 0}, {6, 0, 0}},
 };
+// The entry of kVerts at corner (ci, cj) of a panel, at [panel - 1][2*cj + ci].
+static __constant__ int8_t kVertexAt[6][4] = {{2, 3, 0, 1}, {3, 6, 1, 4}, {6, 7, 4, 5},
+                                              {7, 2, 5, 0}, {0, 1, 5, 4}, {7, 6, 2, 3}};
 
 
 // ---------------------------------------------------------------------------
@@ -352,8 +403,24 @@ __device__ __forceinline__ double ghost_interp(const double *q, double c, double
 // 2x2 apply with M = (m11, m21, m12, m22) (projection_mod.F90:60-96)
 __device__ __forceinline__ void apply2(const double *M, double a, double b, double &o1,
                                        double &o2) {
-  o1 = M[0] * a + M[2] * b;
-  o2 = M[1] * a + M[3] * b;
+  const MCV_GLOBAL double *const m = (const MCV_GLOBAL double *)M;
+  o1 = m[0] * a + m[2] * b;
+  o2 = m[1] * a + m[3] * b;
+}
+
+// The same uniform, read-only struct behind an address the compiler knows
+// nothing about: what it read through the other reference is not kept in
+// scalar registers across the code between the two, but loaded again (scalar
+// loads, constant address space).
+template <typename T>
+__device__ __forceinline__ const T &reread(const T &x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  auto p = (const __attribute__((address_space(4))) T *)&x;
+  asm volatile("" : "+s"(p));
+  return *(const T *)p;
+#else
+  return x;
+#endif
 }
 
 // blockIdx -> logical work index so that the blocks one XCD runs are

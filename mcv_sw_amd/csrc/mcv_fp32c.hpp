@@ -30,14 +30,16 @@ namespace mcv {
 struct MeshF32 {
   int dof, n, npv, nh;
   double rdx, r2dx, rdxx;       // 1/dx, 1/(2 dx), 1/dx^2
-  double dxf;                   // dx
+  double dx;
   long long metric_pstride;
-  const double *sg, *rsg, *ig11, *ig12, *ig22;  // FP64 metric (same arrays as the FP64 path)
-  const D2 *mpack, *spack;      // the same terms packed per point (MeshDev::mpack, spack)
+  const D2 *mpack;              // FP64 metric terms (MeshDev::mpack)
   const double *pgref;          // phi_ref * sqrtG (FP64: a rounded copy is a fixed mass-flux error)
   // {dE/dx, dE/dy, f, 0}: RN32 of the FP64 MCV derivatives (x, y) of
   // phi_ref + phi_s and of the Coriolis parameter, one 16-byte load
   const F4 *fdE;
+  // tables of the boundary pass (MeshDev)
+  const double *p2sp, *sp2p_ghost, *sp2p_edge, *gcoef;
+  const int32_t *giref;
 };
 
 struct StageArgs32 {
@@ -48,8 +50,11 @@ struct StageArgs32 {
   F3 *acc;                                 // RK4 accumulator
   F3 *o;                                   // stage output (raw interior)
   F3 *oc;                                  // compensation of the output (last stage only)
-  F3 *band_raw;                            // raw band lines (hi), see band_point()
-  F3 *band_raw_c;                          // raw band lines (lo), last stage only
+  D3 *band_raw;                            // raw band lines (FP64, hi + lo in the last stage)
+  const D3 *band_in;                       // the band of the stage that wrote `in`
+  // level whose edge lines a raw input's owners finish: `in`, where this stage
+  // (its phi') or a later one reads it again, or null; and its compensation
+  F3 *fin, *fin_c;
   double c1;                               // stage increment coefficient (x dt)
 };
 
@@ -92,12 +97,56 @@ __device__ __forceinline__ T cell_interior_t(const T *f, T dL, T dR, int pos, T 
   }
 }
 
-// One (panel p, tile tx, ty) of the FP32C operator + RK stage `kind`; LDS of
-// at least TileLayout<FP32CStencil, DOF, CX, CY>::kBytes.
+// A level's FP32 values of x and the FP32 residues (Kahan words) beside them.
+__device__ __forceinline__ F3 high_part(const D3 &x) {
+  return F3{(float)x.a, (float)x.b, (float)x.c};
+}
+__device__ __forceinline__ F3 residue(const D3 &x, const F3 &hi) {
+  return F3{(float)(x.a - (double)hi.a), (float)(x.b - (double)hi.b), (float)(x.c - (double)hi.c)};
+}
+
+// As finish_side_points, on an FP32C level.
 template <int DOF, int CX, int CY>
-__device__ __forceinline__ void stage_tile_f32(const MeshF32 &m, const StageArgs32 &a,
-                                               const int kind, const int p, const int tx,
-                                               const int ty, char *smem) {
+__device__ __forceinline__ bool finish_side_points_f32(const MeshF32 &m, const StageArgs32 &a,
+                                                       const int p, const int tx, const int ty,
+                                                       char *smem) {
+  using TL = TileLayout<FP32CStencil, DOF, CX, CY>;
+  constexpr int H = DOF - 1;
+  constexpr int TX = TL::TX, L = TL::TX > TL::TY ? TL::TX : TL::TY;
+  const int npv = m.npv, nh = m.nh, N = m.n;
+  const int cx0 = tx * CX, cy0 = ty * CY;
+  const int ncx = min(CX, N - cx0), ncy = min(CY, N - cy0);
+  const int i0 = cx0 * H + 1, j0 = cy0 * H + 1;
+  const int nx = ncx * H + 1, ny = ncy * H + 1;
+  const TileSides ts = tile_sides(i0, j0, nx + 2 * H, ny + 2 * H, H, npv);
+  if (__builtin_expect(ts.n == 0, 1)) return false;
+  const int TXo = ncx * H + (cx0 + ncx == N ? 1 : 0);
+  const int TYo = ncy * H + (cy0 + ncy == N ? 1 : 0);
+  const uint32_t pb12 = 12u * (uint32_t)(p - 1) * (uint32_t)(nh * nh), nh12 = 12u * (uint32_t)nh;
+  const TL lds(smem);
+  FP32CStencil *const sU = lds.sU, *const sV = lds.sV, *const sPG = lds.sPG;
+  finish_tile<DOF, L>(m, a.band_in, ts, p, i0, j0, nx, ny, [&](int lx, int ly, const D3 &x) {
+    const int li = ly * TX + lx, ox = lx - H, oy = ly - H;
+    const F3 hi = high_part(x);
+    sPG[li] = hi.a;
+    sU[li] = hi.b;
+    sV[li] = hi.c;
+    if (a.fin && ox >= 0 && ox < TXo && oy >= 0 && oy < TYo) {
+      const uint32_t gb = pb12 + mul24(j0 - 1 + ly, nh12) + mul24(i0 - 1 + lx, 12u);
+      stgb(a.fin, gb, hi);
+      if (a.fin_c) stgb(a.fin_c, gb, residue(x, hi));
+    }
+  });
+  __syncthreads();
+  return true;
+}
+
+// One (panel p, tile tx, ty) of the FP32C operator + RK stage `kind`; LDS of
+// at least TileLayout<FP32CStencil, DOF, CX, CY>::kBytes.  `at_side` as in stage_body.
+template <int DOF, int CX, int CY>
+__device__ __forceinline__ void stage_body_f32(const MeshF32 &m, const StageArgs32 &a,
+                                               const int kind, const bool at_side, const int p,
+                                               const int tx, const int ty, char *smem) {
   using C = FP32CStencil;
   using TL = TileLayout<C, DOF, CX, CY>;
   constexpr int H = DOF - 1;
@@ -109,7 +158,7 @@ __device__ __forceinline__ void stage_tile_f32(const MeshF32 &m, const StageArgs
           *const rxV = lds.rxV, *const ryF = lds.ryF, *const ryD = lds.ryD, *const ryU = lds.ryU;
 
   const int npv = m.npv, nh = m.nh, N = m.n;
-  const C rdx = (C)m.rdx, r2dx = (C)m.r2dx, rdxx = (C)m.rdxx, dxf = (C)m.dxf;
+  const C rdx = (C)m.rdx, r2dx = (C)m.r2dx, rdxx = (C)m.rdxx, dxf = (C)m.dx;
   const int cx0 = tx * CX, cy0 = ty * CY;
   const int ncx = min(CX, N - cx0), ncy = min(CY, N - cy0);
   const int i0 = cx0 * H + 1, j0 = cy0 * H + 1;
@@ -126,61 +175,74 @@ __device__ __forceinline__ void stage_tile_f32(const MeshF32 &m, const StageArgs
   const uint32_t pb12 = 12u * pbase, nh12 = 12u * (uint32_t)nh;
   auto rec = [&](int row, int col) { return pb12 + mul24(row, nh12) + mul24(col, 12u); };
 
+  // the points that finish_side_points has left in LDS: ghost points and edge lines
+  auto finished = [&](int lx, int ly) {
+    const int i = i0 - H + lx, j = j0 - H + ly;
+    return i <= 1 || i >= npv || j <= 1 || j >= npv;
+  };
+
   // loads of all a thread's points first, then the derived values
-  constexpr int kP0 = (TX * TY + kStageThreads - 1) / kStageThreads;
-  for (int t0 = threadIdx.x; t0 < TX * TY; t0 += kP0 * blockDim.x) {
-    F3 rs[kP0];
-    double rpg[kP0];
-    double r11[kP0], r12[kP0], r22[kP0], rsg[kP0];
-    bool live[kP0];
+  // Tiles without such points have a copy of the loop without the test.
+  auto stage_points = [&](auto at_side) {
+    constexpr bool edge = decltype(at_side)::value;
+    constexpr int kP0 = (TX * TY + kStageThreads - 1) / kStageThreads;
+    for (int t0 = threadIdx.x; t0 < TX * TY; t0 += kP0 * blockDim.x) {
+      F3 rs[kP0];
+      double rpg[kP0];
+      double r11[kP0], r12[kP0], r22[kP0], rsg[kP0];
+      bool live[kP0];
 #pragma unroll
-    for (int q = 0; q < kP0; ++q) {
-      const int t = t0 + q * blockDim.x;
-      const int ly = div_small<TX>(t), lx = t - ly * TX;
-      const bool inx = lx >= H && lx < H + nx, iny = ly >= H && ly < H + ny;
-      live[q] = t < TX * TY && lx < lw && ly < lh && (inx || iny);
-      if (!live[q]) continue;
-      const uint32_t off = mul24(j0 - 1 + ly, nh) + (uint32_t)(i0 - 1 + lx);
-      const uint32_t g = pbase + off;
-      rs[q] = ldgb(a.in, rec(j0 - 1 + ly, i0 - 1 + lx));
-      rpg[q] = ldg(m.pgref, g);
-      const D2 ga = ldg(mpk, 2 * off), gb = ldg(mpk, 2 * off + 1);
-      rsg[q] = ga.a;
-      r11[q] = ga.b;
-      r12[q] = gb.a;
-      r22[q] = gb.b;
-    }
+      for (int q = 0; q < kP0; ++q) {
+        const int t = t0 + q * blockDim.x;
+        const int ly = div_small<TX>(t), lx = t - ly * TX;
+        const bool inx = lx >= H && lx < H + nx, iny = ly >= H && ly < H + ny;
+        live[q] = t < TX * TY && lx < lw && ly < lh && (inx || iny);
+        if (!live[q]) continue;
+        const uint32_t off = mul24(j0 - 1 + ly, nh) + (uint32_t)(i0 - 1 + lx);
+        const uint32_t g = pbase + off;
+        if (edge && finished(lx, ly)) rs[q] = F3{(float)sPG[t], (float)sU[t], (float)sV[t]};
+        else rs[q] = ldgb(a.in, rec(j0 - 1 + ly, i0 - 1 + lx));
+        rpg[q] = ldg(m.pgref, g);
+        const D2 ga = ldg(mpk, 2 * off), gb = ldg(mpk, 2 * off + 1);
+        rsg[q] = ga.a;
+        r11[q] = ga.b;
+        r12[q] = gb.a;
+        r22[q] = gb.b;
+      }
 #pragma unroll
-    for (int q = 0; q < kP0; ++q) {
-      if (!live[q]) continue;
-      const int li = t0 + q * blockDim.x;  // = ly * TX + lx
-      const int ly = div_small<TX>(li), lx = li - ly * TX;
-      const float dp = rs[q].a, u = rs[q].b, v = rs[q].c;
-      // metric products in FP64 (the FP32 inputs are exact in FP64), rounded once
-      const double ud = u, vd = v;
-      const double g11 = r11[q], g12 = r12[q], g22 = r22[q];
-      const double cud = g11 * ud + g12 * vd, cvd = g12 * ud + g22 * vd;
-      const double Kd = 0.5 * (cud * ud + cvd * vd);
-      const C pg = (C)(rpg[q] + (double)dp * rsg[q]);
-      const C cu = (C)cud, cv = (C)cvd;
-      sE[li] = (C)((double)dp + Kd);  // E - E_ref
-      sU[li] = u;
-      sV[li] = v;
-      sPG[li] = pg;
-      const bool inx = lx >= H && lx < H + nx, iny = ly >= H && ly < H + ny;
-      if (iny) sCU[TL::cu_at(lx, ly)] = cu;
-      if (inx) sCV[TL::cv_at(lx, ly)] = cv;
-      if (inx && iny) {
-        const int ox = lx - H, oy = ly - H;
-        lds.sSG[TL::core_at(lx, ly)] = rsg[q];
-        // phase 1 forms the wave speeds (one division and square root per cell
-        // end there, two and four per thread here)
-        const int cx = div_small<H>(ox), cy = div_small<H>(oy);
-        if (ox == cx * H) lamx[cx * NY + oy] = (C)g11;
-        if (oy == cy * H) lamy[cy * NX + ox] = (C)g22;
+      for (int q = 0; q < kP0; ++q) {
+        if (!live[q]) continue;
+        const int li = t0 + q * blockDim.x;  // = ly * TX + lx
+        const int ly = div_small<TX>(li), lx = li - ly * TX;
+        const float dp = rs[q].a, u = rs[q].b, v = rs[q].c;
+        // metric products in FP64 (the FP32 inputs are exact in FP64), rounded once
+        const double ud = u, vd = v;
+        const double g11 = r11[q], g12 = r12[q], g22 = r22[q];
+        const double cud = g11 * ud + g12 * vd, cvd = g12 * ud + g22 * vd;
+        const double Kd = 0.5 * (cud * ud + cvd * vd);
+        const C pg = (C)(rpg[q] + (double)dp * rsg[q]);
+        const C cu = (C)cud, cv = (C)cvd;
+        sE[li] = (C)((double)dp + Kd);  // E - E_ref
+        sU[li] = u;
+        sV[li] = v;
+        sPG[li] = pg;
+        const bool inx = lx >= H && lx < H + nx, iny = ly >= H && ly < H + ny;
+        if (iny) sCU[TL::cu_at(lx, ly)] = cu;
+        if (inx) sCV[TL::cv_at(lx, ly)] = cv;
+        if (inx && iny) {
+          const int ox = lx - H, oy = ly - H;
+          lds.sSG[TL::core_at(lx, ly)] = rsg[q];
+          // phase 1 forms the wave speeds (one division and square root per cell
+          // end there, two and four per thread here)
+          const int cx = div_small<H>(ox), cy = div_small<H>(oy);
+          if (ox == cx * H) lamx[cx * NY + oy] = (C)g11;
+          if (oy == cy * H) lamy[cy * NX + ox] = (C)g22;
+        }
       }
     }
-  }
+  };
+  if (at_side) stage_points(std::true_type{});
+  else stage_points(std::false_type{});
   __syncthreads();
 
   // cell ends: a wavefront works along one direction (see stage_tile)
@@ -416,27 +478,35 @@ __device__ __forceinline__ void stage_tile_f32(const MeshF32 &m, const StageArgs
           u = bu + (2.0 / 3.0) * ((double)sU[li] - bu) + a.c1 * ku;
           v = bv + (2.0 / 3.0) * ((double)sV[li] - bv) + a.c1 * kv;
         }
-        const float hph = (float)ph, hu = (float)u, hv = (float)v;
-        const F3 hi{hph, hu, hv};
+        const F3 hi = high_part(D3{ph, u, v});
         // the rounding residue (Kahan word), kept by the last stage only
-        const F3 lo{(float)(ph - (double)hph), (float)(u - (double)hu), (float)(v - (double)hv)};
+        const F3 lo = residue(D3{ph, u, v}, hi);
         stgb(a.o, gb, hi);
         if (a.oc) stgb(a.oc, gb, lo);
-        // raw band records (and their residues in the last stage) for the boundary pass
+        // raw copy of the lines nearest each side for the boundary pass: the
+        // level's own values, hi or hi + lo, in FP64
         if (i <= H + 1 || i >= npv - H || j <= H + 1 || j >= npv - H) {
-          // one record per side the point is near (a corner point is near two)
-          auto put = [&](uint32_t bp) {
-            stg(a.band_raw, bp, hi);
-            if (a.oc) stg(a.band_raw_c, bp, lo);
-          };
-          if (i <= H + 1) put(band_point(npv, H, p, 0, i, j));
-          if (i >= npv - H) put(band_point(npv, H, p, 1, npv + 1 - i, j));
-          if (j <= H + 1) put(band_point(npv, H, p, 2, j, i));
-          if (j >= npv - H) put(band_point(npv, H, p, 3, npv + 1 - j, i));
+          const double bp = last ? (double)hi.a + (double)lo.a : (double)hi.a;
+          const double bu = last ? (double)hi.b + (double)lo.b : (double)hi.b;
+          const double bv = last ? (double)hi.c + (double)lo.c : (double)hi.c;
+          const size_t g = pbase + mul24(j + H - 1, nh) + (uint32_t)(i + H - 1);
+          put_band(a.band_raw, npv, H, p, i, j, m.p2sp + 4 * g, bp, bu, bv);
         }
       }
     }
   }
+}
+
+// A stage of one tile, as stage_tile.
+template <int DOF, int CX, int CY, bool Reread>
+__device__ __forceinline__ void stage_tile_f32(const MeshF32 &m, const StageArgs32 &a, const int kind,
+                                   const bool raw, const int p, const int tx, const int ty,
+                                   char *smem) {
+  const bool at_side = raw && finish_side_points_f32<DOF, CX, CY>(m, a, p, tx, ty, smem);
+  if constexpr (Reread)
+    stage_body_f32<DOF, CX, CY>(reread(m), reread(a), kind, at_side, p, tx, ty, smem);
+  else
+    stage_body_f32<DOF, CX, CY>(m, a, kind, at_side, p, tx, ty, smem);
 }
 
 template <int DOF, int KIND, int CX, int CY>
@@ -445,118 +515,40 @@ __global__ __launch_bounds__(kStageThreads) void stage_kernel_f32(MeshF32 m, Sta
   __shared__ __align__(16) char smem[TileLayout<FP32CStencil, DOF, CX, CY>::kBytes];
   const int L = xcd_remap(blockIdx.x, gridDim.x);
   const int tile = L / 6;
-  stage_tile_f32<DOF, CX, CY>(m, a, KIND, L % 6 + 1, tile % tiles_x, tile / tiles_x, smem);
+  stage_body_f32<DOF, CX, CY>(m, a, KIND, false, L % 6 + 1, tile % tiles_x, tile / tiles_x, smem);
+}
+
+// The same on a raw input.
+template <int DOF, int KIND, int CX, int CY>
+__global__ __launch_bounds__(kStageThreads, (stage_waves<FP32CStencil, DOF, CX, CY>())) void
+stage_kernel_raw_f32(StageLaunch<MeshF32, StageArgs32> args) {
+  __shared__ __align__(16) char smem[TileLayout<FP32CStencil, DOF, CX, CY>::kBytes];
+  const StageLaunch<MeshF32, StageArgs32> &k = launch_args(args);
+  const int L = xcd_remap(blockIdx.x, gridDim.x);
+  const int tile = L / 6, tiles_x = k.tiles_x;
+  stage_tile_f32<DOF, CX, CY, true>(k.m, k.a, KIND, true, L % 6 + 1, tile % tiles_x,
+                                    tile / tiles_x, smem);
 }
 
 // correct_bdy_ghost on an FP32C level: same algorithm as the FP64 boundary
 // kernel, values in FP32 storage, arithmetic and ghost weights in FP64.  The
 // deviation phi' is interpolated and averaged like phi (both operations are
 // linear and phi_ref is already continuous across edges).  For the base state
-// (cpu != NULL) values are hi + lo and every written point gets its residue.
+// (comp != NULL) the band holds hi + lo and every written point gets its residue.
 struct BoundaryArgs32 {
   F3 *lev;                 // level to finish: {phi', u, v} records
   F3 *comp;                // its compensation words (base state only, else NULL)
-  const F3 *band_raw, *band_raw_c;  // raw band records; residues for the base state
+  const D3 *band_raw;
 };
 
 template <int DOF>
-__device__ __forceinline__ void boundary_item_f32(const MeshDev &m, const BoundaryArgs32 &ba,
+__device__ __forceinline__ void boundary_item_f32(const MeshDev &m, const BoundaryArgs32 &a,
                                                   const int t) {
-  constexpr int H = DOF - 1;
-  F3 *const lev = ba.lev, *const comp = ba.comp;
-  const int npv = m.npv, nh = m.nh;
-  const double dx = m.dx;
-  const int nghost = 6 * 4 * H * npv, nedge = 12 * npv;
-  // raw value of band point (panel q, side, depth d, along index al): hi, plus
-  // lo for the base state
-  auto raw = [&](int q, int side, int d, int al, double &ph, double &uu, double &vv) {
-    const uint32_t bp = band_point(npv, H, q, side, d, al);
-    const F3 r = ldg(ba.band_raw, bp);
-    ph = r.a; uu = r.b; vv = r.c;
-    if (comp) {
-      const F3 c = ldg(ba.band_raw_c, bp);
-      ph += (double)c.a;
-      uu += (double)c.b;
-      vv += (double)c.c;
-    }
-  };
-  auto store = [&](long long g, double ph, double uu, double vv) {
-    const float a0 = (float)ph, a1 = (float)uu, a2 = (float)vv;
-    lev[g] = F3{a0, a1, a2};
-    if (comp) comp[g] = F3{(float)(ph - (double)a0), (float)(uu - (double)a1), (float)(vv - (double)a2)};
-  };
-  if (t < nghost) {  // one ghost point: (panel, side, depth k, s), s fastest
-    const int s = t % npv + 1, r = t / npv, k = r % H + 1, ps = r / H;
-    const int side = ps % 4, p = ps / 4 + 1;
-    const HaloSrc hs = kHalo[p - 1][side];
-    const int src = hs.col ? (hs.far ? 1 : 0) : (hs.far ? 3 : 2);
-    const int c = m.giref[(k - 1) * npv + (s - 1)];
-    const double cf = m.gcoef[(k - 1) * npv + (s - 1)];
-    double qp[DOF], qz[DOF], qm[DOF];
-    for (int l = 0; l < DOF; ++l) {
-      const int tpos = (c - 1) * H + 1 + l;
-      const int al = hs.rev ? npv + 1 - tpos : tpos;
-      double ph, uu, vv;
-      raw(hs.q, src, k + 1, al, ph, uu, vv);
-      qp[l] = ph;
-      apply2(m.p2sp_band + 4 * band_point(npv, H, hs.q, src, k + 1, al), uu, vv, qz[l], qm[l]);
-    }
-    int hi, hj;
-    if (side == 0) { hi = 1 - k; hj = s; }
-    else if (side == 1) { hi = npv + k; hj = s; }
-    else if (side == 2) { hi = s; hj = 1 - k; }
-    else { hi = s; hj = npv + k; }
-    const long long g = pidx(nh, H, p, hi, hj);
-    const double zh = ghost_interp<DOF>(qz, cf, dx), mh = ghost_interp<DOF>(qm, cf, dx);
-    double uh, vh;
-    apply2(m.sp2p_ghost + 4 * ghost_point(npv, H, p, side, k, s), zh, mh, uh, vh);
-    store(g, ghost_interp<DOF>(qp, cf, dx), uh, vh);
-  } else if (t < nghost + nedge) {  // one point of one cube edge
-    const int s = (t - nghost) % npv + 1, e = (t - nghost) / npv;
-    if (s > 1 && s < npv) {
-      const EdgePair ep = kEdges[e];
-      const int sb = ep.rev ? npv + 1 - s : s;
-      int ia, ja, ib, jb;
-      edge_ij(npv, ep.sa, s, ia, ja);
-      edge_ij(npv, ep.sb, sb, ib, jb);
-      const long long ga = pidx(nh, H, ep.pa, ia, ja), gb = pidx(nh, H, ep.pb, ib, jb);
-      double pa, ua, va, pb, ub, vb;
-      raw(ep.pa, ep.sa, 1, s, pa, ua, va);
-      raw(ep.pb, ep.sb, 1, sb, pb, ub, vb);
-      double za, ma, zb, mb;
-      apply2(m.p2sp_band + 4 * band_point(npv, H, ep.pa, ep.sa, 1, s), ua, va, za, ma);
-      apply2(m.p2sp_band + 4 * band_point(npv, H, ep.pb, ep.sb, 1, sb), ub, vb, zb, mb);
-      const double ph = 0.5 * (pa + pb), zu = 0.5 * (za + zb), mu = 0.5 * (ma + mb);
-      double u1, v1, u2, v2;
-      apply2(m.sp2p_edge + 4 * edge_point(npv, ep.pa, ep.sa, s), zu, mu, u1, v1);
-      apply2(m.sp2p_edge + 4 * edge_point(npv, ep.pb, ep.sb, sb), zu, mu, u2, v2);
-      store(ga, ph, u1, v1);
-      store(gb, ph, u2, v2);
-    }
-  } else {
-    const int vx = t - nghost - nedge;
-    double ph[3], z[3], mr[3];
-    long long gg[3];
-    uint32_t eg[3];
-    for (int l = 0; l < 3; ++l) {
-      const VtxPt vp = kVerts[vx][l];
-      const int i = vp.ci ? npv : 1, j = vp.cj ? npv : 1;
-      const int side = vp.ci ? 1 : 0;
-      double uu, vv;
-      raw(vp.p, side, 1, j, ph[l], uu, vv);
-      gg[l] = pidx(nh, H, vp.p, i, j);
-      eg[l] = edge_point(npv, vp.p, side, j);
-      apply2(m.p2sp_band + 4 * band_point(npv, H, vp.p, side, 1, j), uu, vv, z[l], mr[l]);
-    }
-    const double pv = (ph[0] + ph[1] + ph[2]) / 3.0;
-    const double zv = (z[0] + z[1] + z[2]) / 3.0;
-    const double mv = (mr[0] + mr[1] + mr[2]) / 3.0;
-    for (int l = 0; l < 3; ++l) {
-      double uu, vv;
-      apply2(m.sp2p_edge + 4 * eg[l], zv, mv, uu, vv);
-      store(gg[l], pv, uu, vv);
-    }
-  }
+  boundary_item<DOF>(m, a.band_raw, t, [&](long long g, const D3 &x) {
+    const F3 hi = high_part(x);
+    write_global((MCV_GLOBAL char *)(a.lev + g), hi);
+    if (a.comp) write_global((MCV_GLOBAL char *)(a.comp + g), residue(x, hi));
+  });
 }
 
 template <int DOF>
@@ -576,9 +568,8 @@ static __global__ void pgref_kernel(MeshDev m, const double *phi_ref, double *pg
   }
 }
 
-// FP64 band copy of a finished level (to run the boundary pass on it).
-static __global__ void band_copy_kernel(MeshDev m, const D2 *pu, const double *v,
-                                        double *band) {
+// Band of a finished level (to run the boundary pass on it).
+static __global__ void band_copy_kernel(MeshDev m, const D2 *pu, const double *v, D3 *band) {
   const int npv = m.npv, H = m.dof - 1;
   const int n = 6 * 4 * (H + 1) * npv;
   for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < n; t += gridDim.x * blockDim.x) {
@@ -588,9 +579,9 @@ static __global__ void band_copy_kernel(MeshDev m, const D2 *pu, const double *v
     band_ij(npv, side, d, al, i, j);
     const long long g = pidx(m.nh, H, p, i, j);
     const D2 x = pu[g];
-    band[band_slot(npv, H, p, side, d, 0, al)] = x.a;
-    band[band_slot(npv, H, p, side, d, 1, al)] = x.b;
-    band[band_slot(npv, H, p, side, d, 2, al)] = v[g];
+    D3 &o = band[band_point(npv, H, p, side, d, al)];
+    o.a = x.a;
+    apply2(m.p2sp + 4 * g, x.b, v[g], o.b, o.c);
   }
 }
 

@@ -52,15 +52,53 @@ template <> struct TileSet32<4> {
   static constexpr int cy[kTileVariants] = {4, 4, 8, 6};
 };
 
+// Where the boundary pass runs: inside the next stage's kernel (its side tiles
+// finish the points they stage) or in a launch of its own after each stage.
+// The launch costs a dispatch and a drained chip, which dominates small work;
+// inside, the side tiles live longer and drag on launches that fill the chip
+// several times over.  The pass is built into the kernels of the two small tile
+// shapes of each order, which small work takes.
+// The limit, 18 tiles per CU, from both sides measured (us per step, launch of
+// its own / inside): MCV3 6x32^2 FP64 RK4 38.4 / 29.1, 6x90^2 FP32C RK3 (972
+// tiles) 30.2 / 26.9, MCV4 6x96^2 FP64 (2400) 91.7 / 88.0, MCV3 6x181^2 FP64 RK3
+// (4218) 74.0 / 69.5, MCV4 6x160^2 FP64 (6144) 177.5 / 178.2, 6x384^2 FP32C
+// 730 / 782; MCV3 6x90^2 FP32C ensembles per stage, 1 member 12.6 / 11.0, 4
+// members (3888) 25.4 / 25.0, 6 members (5832) 32.0 / 32.8, 20 members 99.5 / 103.9.
+constexpr int kFusedMaxTiles = 18 * 256;
+inline bool sides_in_stage(int tile_variant, long long tiles) {
+  return (tile_variant == 0 || tile_variant == 2) && tiles <= kFusedMaxTiles;
+}
+
 // Upper bound of the device bytes one solve of this configuration allocates
 // (exact when the metric terms differ between panels).
 size_t footprint_bytes(const mcv_config *c);
 
-// Stage and boundary arguments of a solve's levels (level 0 is Y_n).
-StageArgs stage_args64(const mcv_handle *h, int in, int out, double c1);
-StageArgs32 stage_args32(const mcv_handle *h, int in, int out, double c1);
-BoundaryArgs boundary_args64(const mcv_handle *h, int level);
-BoundaryArgs32 boundary_args32(const mcv_handle *h, int level);
+// The RK stages of a time step (time_scheme_mod.F90:13-69).  Levels: 0 = Yn
+// (updated in place by the last stage), 1 and 2 = intermediate stage states.
+// Each stage writes a band of its own and reads the one before it, which other
+// workgroups of the same launch may still be reading: RK4 alternates between
+// two bands, RK3, with its odd number of stages, goes round three.
+struct StageSpec {
+  int kind, in, out;
+  double c1;  // stage increment coefficient (x dt)
+};
+inline int stage_count(int scheme) { return scheme == MCV_RK4 ? 4 : 3; }
+inline int band_count(int scheme) { return scheme == MCV_RK4 ? 2 : 3; }
+inline StageSpec stage_spec(const mcv_config &c, int s) {
+  const double dt = c.dt;
+  const StageSpec rk4[4] = {{kRK4S1, 0, 1, 0.5 * dt}, {kRK4S2, 1, 2, 0.5 * dt},
+                            {kRK4S3, 2, 1, dt}, {kRK4S4, 1, 0, dt}};
+  const StageSpec rk3[3] = {{kRK3S1, 0, 1, dt}, {kRK3S2, 1, 2, 0.25 * dt},
+                            {kRK3S3, 2, 0, 2.0 / 3.0 * dt}};
+  return c.scheme == MCV_RK4 ? rk4[s] : rk3[s];
+}
+
+// Arguments of stage s of a solve's time step, and of the boundary pass on the
+// level it wrote.
+StageArgs stage_args64(const mcv_handle *h, int s);
+StageArgs32 stage_args32(const mcv_handle *h, int s);
+BoundaryArgs boundary_args64(const mcv_handle *h, int s);
+BoundaryArgs32 boundary_args32(const mcv_handle *h, int s);
 
 }  // namespace mcv
 
@@ -77,7 +115,7 @@ struct mcv_handle {
   double *lvv[3] = {};         //   and v
   double *phi_ref = nullptr;   // FP32C: the projected initial geopotential (FP64)
   double *acc[3] = {};         // RK4 accumulator: acc[0] {phiG, u} pairs, acc[2] v
-  double *band_raw = nullptr;  // raw band lines written by the stage kernel
+  mcv::D3 *band_raw[3] = {};   // raw band lines written by the stage kernel
   double *cu0 = nullptr, *cv0 = nullptr;  // host contra winds until the first stage
   bool first_pending = true;
   double *partials = nullptr;
@@ -102,7 +140,6 @@ struct mcv_handle {
   mcv::F3 *l32[3] = {};
   mcv::F3 *c32 = nullptr;
   mcv::F3 *a32 = nullptr;
-  mcv::F3 *band32 = nullptr, *band32c = nullptr;  // FP32 band records and residues
   double *join[3] = {};  // FP64 reconstruction of Y_n for read-back and integrals
   mcv::MeshF32 mesh32{};
 };

@@ -35,64 +35,75 @@ int fail(int code, const char *fmt, ...) {
 
 size_t footprint_bytes(const mcv_config *c) {
   const size_t H = c->dof - 1, npv = (size_t)c->n * H + 1, nh = npv + 2 * H;
-  const size_t np = 6 * nh * nh, nband = band_values(c->dof, (int)npv), pad = 256;
+  const size_t np = 6 * nh * nh, nband = 3 * band_points(c->dof, (int)npv), pad = 256;
   const size_t ncell = 6 * (size_t)c->n * c->n;
   const size_t diag_blocks =
       std::min<size_t>((ncell + kDiagThreads - 1) / kDiagThreads, kDiagMaxBlocks);
   auto d = [&](size_t count) { return count * sizeof(double) + pad; };
   auto f = [&](size_t count) { return count * sizeof(float) + pad; };
   // static mesh data (panel-invariant metric terms counted on every panel)
-  size_t b = 5 * d(np) + d(np) + d(np) + d(4 * np) + d(H * npv) +
+  size_t b = 4 * d(np) + d(np) + d(np) + d(4 * np) + d(H * npv) +
              sizeof(int32_t) * H * npv + pad;
-  b += d(4 * np) + d(2 * np);  // packed metric terms
-  b += d(4 * 6 * 4 * (H + 1) * npv) + d(4 * 6 * 4 * H * npv) + d(4 * 6 * 4 * npv);  // band tables
+  b += d(4 * np);  // packed metric terms
+  b += d(4 * 6 * 4 * H * npv) + d(4 * 6 * 4 * npv);  // tables of the boundary pass
   const bool fp32c = c->precision == MCV_FP32C;
   b += (fp32c ? 3 : 9) * d(np);                       // FP64 levels
   if (!fp32c) b += 3 * d(np);                          // RK4 accumulator
-  b += d(nband) + 2 * d(np) + d(4 * diag_blocks) + d(2) + 6 * d(np);
+  b += band_count(c->scheme) * d(nband) + 2 * d(np) + d(4 * diag_blocks) + d(2) + 6 * d(np);
   if (fp32c)  // join, phi_ref, phi_ref*sqrtG, FP32 {reference gradient, Coriolis, 0},
-              // levels, compensation, accumulator, bands
-    b += 3 * d(np) + d(np) + d(np) + 4 * f(np) + 3 * f(3 * np) + f(3 * np) + f(3 * np) +
-         2 * f(nband);
+              // levels, compensation, accumulator
+    b += 3 * d(np) + d(np) + d(np) + 4 * f(np) + 3 * f(3 * np) + f(3 * np) + f(3 * np);
   return b;
 }
 
-StageArgs stage_args64(const mcv_handle *h, int in, int out, double c1) {
+StageArgs stage_args64(const mcv_handle *h, int s) {
+  const StageSpec sp = stage_spec(h->cfg, s);
+  const int nst = stage_count(h->cfg.scheme), nb = band_count(h->cfg.scheme);
   StageArgs a{};
-  a.in_pu = h->lpu[in]; a.in_v = h->lvv[in];
+  a.in_pu = h->lpu[sp.in]; a.in_v = h->lvv[sp.in];
   a.b_pu = h->lpu[0]; a.b_v = h->lvv[0];
   a.acc_pu = reinterpret_cast<D2 *>(h->acc[0]); a.acc_v = h->acc[2];
-  a.o_pu = h->lpu[out]; a.o_v = h->lvv[out];
-  a.band_raw = h->band_raw;
-  a.c1 = c1;
+  a.o_pu = h->lpu[sp.out]; a.o_v = h->lvv[sp.out];
+  a.band_raw = h->band_raw[s % nb];
+  a.band_in = h->band_raw[(s + nst - 1) % nst % nb];
+  if (s == 0) { a.fin_pu = h->lpu[0]; a.fin_v = h->lvv[0]; }
+  a.c1 = sp.c1;
   return a;
 }
 
-BoundaryArgs boundary_args64(const mcv_handle *h, int level) {
-  return BoundaryArgs{h->lpu[level], h->lvv[level], h->band_raw};
+BoundaryArgs boundary_args64(const mcv_handle *h, int s) {
+  const int out = stage_spec(h->cfg, s).out;
+  return BoundaryArgs{h->lpu[out], h->lvv[out], h->band_raw[s % band_count(h->cfg.scheme)]};
 }
 
-StageArgs32 stage_args32(const mcv_handle *h, int in, int out, double c1) {
+StageArgs32 stage_args32(const mcv_handle *h, int s) {
+  const StageSpec sp = stage_spec(h->cfg, s);
+  const int nst = stage_count(h->cfg.scheme), nb = band_count(h->cfg.scheme);
   StageArgs32 a{};
-  a.in = h->l32[in];
+  a.in = h->l32[sp.in];
   a.b = h->l32[0];
   a.c = h->c32;
   a.acc = h->a32;
-  a.o = h->l32[out];
-  if (out == 0) a.oc = h->c32;  // the step's last stage writes Y_n+1 with its compensation
-  a.band_raw = h->band32;
-  a.band_raw_c = h->band32c;
-  a.c1 = c1;
+  a.o = h->l32[sp.out];
+  if (sp.out == 0) a.oc = h->c32;  // the step's last stage writes Y_n+1 with its compensation
+  a.band_raw = h->band_raw[s % nb];
+  a.band_in = h->band_raw[(s + nst - 1) % nst % nb];
+  if (s == 0) {  // Y_n, raw from the step before: base of the stages that follow
+    a.fin = h->l32[0];
+    a.fin_c = h->c32;
+  } else if (h->cfg.scheme == MCV_RK3_TVD) {  // the update reads phi' of its input
+    a.fin = h->l32[sp.in];
+  }
+  a.c1 = sp.c1;
   return a;
 }
 
-BoundaryArgs32 boundary_args32(const mcv_handle *h, int level) {
-  const bool base = level == 0;  // Y_n carries its compensation words
+BoundaryArgs32 boundary_args32(const mcv_handle *h, int s) {
+  const int out = stage_spec(h->cfg, s).out;
   BoundaryArgs32 b{};
-  b.lev = h->l32[level];
-  if (base) b.comp = h->c32;
-  b.band_raw = h->band32;
-  b.band_raw_c = h->band32c;
+  b.lev = h->l32[out];
+  if (out == 0) b.comp = h->c32;  // Y_n carries its compensation words
+  b.band_raw = h->band_raw[s % band_count(h->cfg.scheme)];
   return b;
 }
 
@@ -142,6 +153,19 @@ int dev_alloc(mcv_handle *h, double **out, size_t count) {
   return MCV_OK;
 }
 
+template <typename T>
+int dev_alloc_t(mcv_handle *h, T **out, size_t count) {
+  void *p = nullptr;
+  hipError_t e = hipMalloc(&p, count * sizeof(T) + 256);
+  if (e != hipSuccess)
+    return fail(MCV_ENOMEM, "hipMalloc(%zu bytes) failed: %s", count * sizeof(T),
+                hipGetErrorString(e));
+  h->allocs.push_back(p);
+  h->device_bytes += count * sizeof(T) + 256;
+  *out = static_cast<T *>(p);
+  return MCV_OK;
+}
+
 int upload(mcv_handle *h, double **dst, const double *src, size_t count) {
   int rc = dev_alloc(h, dst, count);
   if (rc) return rc;
@@ -187,15 +211,40 @@ int validate(const mcv_config *c) {
   return MCV_OK;
 }
 
-template <int DOF, int CX, int CY>
-int launch_stage_shape(mcv_handle *h, int kind, const StageArgs &a) {
+template <int DOF, int V>
+int launch_stage_shape(mcv_handle *h, int kind, const StageArgs &a, bool raw) {
+  constexpr int CX = TileSet<DOF>::cx[V], CY = TileSet<DOF>::cy[V];
   const int tx = (h->cfg.n + CX - 1) / CX, ty = (h->cfg.n + CY - 1) / CY;
   dim3 grid(tx * ty * 6), block(kStageThreads);
+  if (raw) {
+    if constexpr (V == 0 || V == 2) {
+      const StageLaunch<MeshDev, StageArgs> args{h->mesh, a, tx};
+      switch (kind) {
+#define MCV_CASE(K)                                                                            \
+  case K:                                                                                      \
+    hipLaunchKernelGGL((stage_kernel_raw<DOF, K, CX, CY>), grid, block, 0, h->stream, args); \
+    break;
+    MCV_CASE(kRK4S1)
+    MCV_CASE(kRK4S2)
+    MCV_CASE(kRK4S3)
+    MCV_CASE(kRK4S4)
+    MCV_CASE(kRK3S1)
+    MCV_CASE(kRK3S2)
+    MCV_CASE(kRK3S3)
+#undef MCV_CASE
+        default:
+          return fail(MCV_EINVAL, "bad stage kind %d", kind);
+      }
+      HIP_TRY(hipGetLastError());
+      return MCV_OK;
+    }
+    return fail(MCV_EINVAL, "tile shape %d takes finished levels only", V);
+  }
   switch (kind) {
-#define MCV_CASE(K)                                                                   \
-  case K:                                                                             \
+#define MCV_CASE(K)                                                                        \
+  case K:                                                                                  \
     hipLaunchKernelGGL((stage_kernel<DOF, K, CX, CY>), grid, block, 0, h->stream, h->mesh, \
-                       a, tx);                                                        \
+                       a, tx);                                                             \
     break;
     MCV_CASE(kTend)
     MCV_CASE(kRK4S1)
@@ -214,22 +263,20 @@ int launch_stage_shape(mcv_handle *h, int kind, const StageArgs &a) {
 }
 
 template <int DOF>
-int launch_stage(mcv_handle *h, int kind, const StageArgs &a) {
-  using T = TileSet<DOF>;
+int launch_stage(mcv_handle *h, int kind, const StageArgs &a, bool raw) {
   switch (h->tile) {
-    case 0: return launch_stage_shape<DOF, T::cx[0], T::cy[0]>(h, kind, a);
-    case 1: return launch_stage_shape<DOF, T::cx[1], T::cy[1]>(h, kind, a);
-    case 2: return launch_stage_shape<DOF, T::cx[2], T::cy[2]>(h, kind, a);
-    default: return launch_stage_shape<DOF, T::cx[3], T::cy[3]>(h, kind, a);
+    case 0: return launch_stage_shape<DOF, 0>(h, kind, a, raw);
+    case 1: return launch_stage_shape<DOF, 1>(h, kind, a, raw);
+    case 2: return launch_stage_shape<DOF, 2>(h, kind, a, raw);
+    default: return launch_stage_shape<DOF, 3>(h, kind, a, raw);
   }
 }
 
-int stage(mcv_handle *h, int kind, const StageArgs &a) {
-  return h->cfg.dof == 3 ? launch_stage<3>(h, kind, a) : launch_stage<4>(h, kind, a);
+int stage(mcv_handle *h, int kind, const StageArgs &a, bool raw) {
+  return h->cfg.dof == 3 ? launch_stage<3>(h, kind, a, raw) : launch_stage<4>(h, kind, a, raw);
 }
 
-int boundary(mcv_handle *h, int level) {
-  const BoundaryArgs b = boundary_args64(h, level);
+int boundary(mcv_handle *h, const BoundaryArgs &b) {
   const int threads = boundary_items(h->cfg.dof, h->npv);
   dim3 grid((threads + 255) / 256), block(256);
   if (h->cfg.dof == 3)
@@ -243,15 +290,40 @@ int boundary(mcv_handle *h, int level) {
 // ---------------------------------------------------------------------------
 // FP32C launches
 // ---------------------------------------------------------------------------
-template <int DOF, int CX, int CY>
-int launch_stage32_shape(mcv_handle *h, int kind, const StageArgs32 &a) {
+template <int DOF, int V>
+int launch_stage32_shape(mcv_handle *h, int kind, const StageArgs32 &a, bool raw) {
+  constexpr int CX = TileSet32<DOF>::cx[V], CY = TileSet32<DOF>::cy[V];
   const int tx = (h->cfg.n + CX - 1) / CX, ty = (h->cfg.n + CY - 1) / CY;
-  dim3 grid(tx * ty * 6), block(256);
+  dim3 grid(tx * ty * 6), block(kStageThreads);
+  if (raw) {
+    if constexpr (V == 0 || V == 2) {
+      const StageLaunch<MeshF32, StageArgs32> args{h->mesh32, a, tx};
+      switch (kind) {
+#define MCV_CASE(K)                                                                            \
+  case K:                                                                                      \
+    hipLaunchKernelGGL((stage_kernel_raw_f32<DOF, K, CX, CY>), grid, block, 0, h->stream, args); \
+    break;
+    MCV_CASE(kRK4S1)
+    MCV_CASE(kRK4S2)
+    MCV_CASE(kRK4S3)
+    MCV_CASE(kRK4S4)
+    MCV_CASE(kRK3S1)
+    MCV_CASE(kRK3S2)
+    MCV_CASE(kRK3S3)
+#undef MCV_CASE
+        default:
+          return fail(MCV_EINVAL, "bad stage kind %d", kind);
+      }
+      HIP_TRY(hipGetLastError());
+      return MCV_OK;
+    }
+    return fail(MCV_EINVAL, "tile shape %d takes finished levels only", V);
+  }
   switch (kind) {
-#define MCV_CASE(K)                                                                       \
-  case K:                                                                                 \
-    hipLaunchKernelGGL((stage_kernel_f32<DOF, K, CX, CY>), grid, block, 0, h->stream,      \
-                       h->mesh32, a, tx);                                                 \
+#define MCV_CASE(K)                                                                        \
+  case K:                                                                                  \
+    hipLaunchKernelGGL((stage_kernel_f32<DOF, K, CX, CY>), grid, block, 0, h->stream, h->mesh32, \
+                       a, tx);                                                             \
     break;
     MCV_CASE(kRK4S1)
     MCV_CASE(kRK4S2)
@@ -262,29 +334,28 @@ int launch_stage32_shape(mcv_handle *h, int kind, const StageArgs32 &a) {
     MCV_CASE(kRK3S3)
 #undef MCV_CASE
     default:
-      return fail(MCV_EINVAL, "bad FP32C stage kind %d", kind);
+      return fail(MCV_EINVAL, "bad stage kind %d", kind);
   }
   HIP_TRY(hipGetLastError());
   return MCV_OK;
 }
 
 template <int DOF>
-int launch_stage32(mcv_handle *h, int kind, const StageArgs32 &a) {
-  using T = TileSet32<DOF>;
+int launch_stage32(mcv_handle *h, int kind, const StageArgs32 &a, bool raw) {
   switch (h->tile) {
-    case 0: return launch_stage32_shape<DOF, T::cx[0], T::cy[0]>(h, kind, a);
-    case 1: return launch_stage32_shape<DOF, T::cx[1], T::cy[1]>(h, kind, a);
-    case 2: return launch_stage32_shape<DOF, T::cx[2], T::cy[2]>(h, kind, a);
-    default: return launch_stage32_shape<DOF, T::cx[3], T::cy[3]>(h, kind, a);
+    case 0: return launch_stage32_shape<DOF, 0>(h, kind, a, raw);
+    case 1: return launch_stage32_shape<DOF, 1>(h, kind, a, raw);
+    case 2: return launch_stage32_shape<DOF, 2>(h, kind, a, raw);
+    default: return launch_stage32_shape<DOF, 3>(h, kind, a, raw);
   }
 }
 
-int stage32(mcv_handle *h, int kind, const StageArgs32 &a) {
-  return h->cfg.dof == 3 ? launch_stage32<3>(h, kind, a) : launch_stage32<4>(h, kind, a);
+int stage32(mcv_handle *h, int kind, const StageArgs32 &a, bool raw) {
+  return h->cfg.dof == 3 ? launch_stage32<3>(h, kind, a, raw)
+                         : launch_stage32<4>(h, kind, a, raw);
 }
 
-int boundary32(mcv_handle *h, int level) {
-  const BoundaryArgs32 b = boundary_args32(h, level);
+int boundary32(mcv_handle *h, const BoundaryArgs32 &b) {
   const int threads = boundary_items(h->cfg.dof, h->npv);
   dim3 grid((threads + 255) / 256), block(256);
   if (h->cfg.dof == 3)
@@ -295,45 +366,71 @@ int boundary32(mcv_handle *h, int level) {
   return MCV_OK;
 }
 
-// One RK stage: stage kernel from level `in` (base Yn = level 0) into level
-// `out`, then the boundary pass on `out`.
-int rk_stage(mcv_handle *h, int kind, int in, int out, double c1) {
-  StageArgs a = h->fp32c ? StageArgs{} : stage_args64(h, in, out, c1);
-  if (h->first_pending) { a.cu0 = h->cu0; a.cv0 = h->cv0; }
+// Stage s of a time step.  `raw`: its input is as the stage before left it
+// (the tiles at the panel sides then form its halo and edge lines themselves).
+int rk_stage(mcv_handle *h, int s, bool raw) {
+  const int kind = stage_spec(h->cfg, s).kind;
   if (h->timing) HIP_TRY(hipEventRecord(h->ev[0], h->stream));
-  int rc = h->fp32c ? stage32(h, kind, stage_args32(h, in, out, c1)) : stage(h, kind, a);
+  int rc;
+  if (h->fp32c) {
+    rc = stage32(h, kind, stage_args32(h, s), raw);
+  } else {
+    StageArgs a = stage_args64(h, s);
+    if (h->first_pending) { a.cu0 = h->cu0; a.cv0 = h->cv0; }
+    rc = stage(h, kind, a, raw);
+  }
   if (rc) return rc;
   h->first_pending = false;
-  if (h->timing) HIP_TRY(hipEventRecord(h->ev[1], h->stream));
-  rc = h->fp32c ? boundary32(h, out) : boundary(h, out);
-  if (rc) return rc;
   if (h->timing) {
     // events bracket each kernel on the handle's stream; wait so they can be reused
-    HIP_TRY(hipEventRecord(h->ev[2], h->stream));
-    HIP_TRY(hipEventSynchronize(h->ev[2]));
-    float a_ms = 0.f, b_ms = 0.f;
-    HIP_TRY(hipEventElapsedTime(&a_ms, h->ev[0], h->ev[1]));
-    HIP_TRY(hipEventElapsedTime(&b_ms, h->ev[1], h->ev[2]));
-    h->stage_ms += a_ms;
-    h->boundary_ms += b_ms;
+    HIP_TRY(hipEventRecord(h->ev[1], h->stream));
+    HIP_TRY(hipEventSynchronize(h->ev[1]));
+    float ms = 0.f;
+    HIP_TRY(hipEventElapsedTime(&ms, h->ev[0], h->ev[1]));
+    h->stage_ms += ms;
   }
   return MCV_OK;
 }
 
-// time_scheme_mod.F90:13-69.  Levels: 0 = Yn (updated in place by the last
-// stage), 1 and 2 = intermediate stage states.
-int one_step(mcv_handle *h) {
-  const double dt = h->cfg.dt;
-  int rc;
-  if (h->cfg.scheme == MCV_RK4) {
-    if ((rc = rk_stage(h, kRK4S1, 0, 1, 0.5 * dt))) return rc;
-    if ((rc = rk_stage(h, kRK4S2, 1, 2, 0.5 * dt))) return rc;
-    if ((rc = rk_stage(h, kRK4S3, 2, 1, dt))) return rc;
-    if ((rc = rk_stage(h, kRK4S4, 1, 0, dt))) return rc;
+// The boundary pass on the level that stage s wrote.
+int boundary_pass(mcv_handle *h, int s) {
+  if (h->timing) HIP_TRY(hipEventRecord(h->ev[0], h->stream));
+  const int rc =
+      h->fp32c ? boundary32(h, boundary_args32(h, s)) : boundary(h, boundary_args64(h, s));
+  if (rc) return rc;
+  if (h->timing) {
+    HIP_TRY(hipEventRecord(h->ev[1], h->stream));
+    HIP_TRY(hipEventSynchronize(h->ev[1]));
+    float ms = 0.f;
+    HIP_TRY(hipEventElapsedTime(&ms, h->ev[0], h->ev[1]));
+    h->boundary_ms += ms;
+  }
+  return MCV_OK;
+}
+
+// nsteps time steps.  Y_n is finished when they are enqueued, as a following
+// call and the read-backs expect it.
+int run_steps(mcv_handle *h, int32_t nsteps) {
+  const int nst = stage_count(h->cfg.scheme), t = h->tile;
+  int cx, cy;
+  if (h->fp32c) {
+    cx = h->cfg.dof == 3 ? TileSet32<3>::cx[t] : TileSet32<4>::cx[t];
+    cy = h->cfg.dof == 3 ? TileSet32<3>::cy[t] : TileSet32<4>::cy[t];
   } else {
-    if ((rc = rk_stage(h, kRK3S1, 0, 1, dt))) return rc;
-    if ((rc = rk_stage(h, kRK3S2, 1, 2, 0.25 * dt))) return rc;
-    if ((rc = rk_stage(h, kRK3S3, 2, 0, 2.0 / 3.0 * dt))) return rc;
+    cx = h->cfg.dof == 3 ? TileSet<3>::cx[t] : TileSet<4>::cx[t];
+    cy = h->cfg.dof == 3 ? TileSet<3>::cy[t] : TileSet<4>::cy[t];
+  }
+  const int n = h->cfg.n;
+  const bool fused = sides_in_stage(t, 6LL * ((n + cx - 1) / cx) * ((n + cy - 1) / cy));
+  bool raw = false;  // the next stage's input is as a stage left it
+  for (int32_t k = 0; k < nsteps; ++k) {
+    for (int s = 0; s < nst; ++s) {
+      int rc = rk_stage(h, s, raw);
+      if (rc) return rc;
+      raw = fused && !(k == nsteps - 1 && s == nst - 1);
+      if (!raw && (rc = boundary_pass(h, s))) return rc;
+    }
+    ++h->steps;
   }
   return MCV_OK;
 }
@@ -388,19 +485,6 @@ int run_diag(mcv_handle *h, double *mass, double *energy) {
   return MCV_OK;
 }
 
-template <typename T>
-int dev_alloc_t(mcv_handle *h, T **out, size_t count) {
-  void *p = nullptr;
-  hipError_t e = hipMalloc(&p, count * sizeof(T) + 256);
-  if (e != hipSuccess)
-    return fail(MCV_ENOMEM, "hipMalloc(%zu bytes) failed: %s", count * sizeof(T),
-                hipGetErrorString(e));
-  h->allocs.push_back(p);
-  h->device_bytes += count * sizeof(T) + 256;
-  *out = static_cast<T *>(p);
-  return MCV_OK;
-}
-
 // FP32C set-up from the FP64 initial state in level 0.  One FP64 boundary
 // pass on a copy makes it continuous across panel edges with an interpolated
 // halo; that projected geopotential is the reference phi_ref (kept in level
@@ -409,7 +493,6 @@ int dev_alloc_t(mcv_handle *h, T **out, size_t count) {
 // stage sees the handed-over halo and edges as the FP64 path does.
 int setup32(mcv_handle *h) {
   const long long np = h->np;
-  const size_t nband = band_values(h->cfg.dof, h->npv);
   const int threads = 6 * 4 * h->cfg.dof * h->npv;
   int rc;
   for (int f = 0; f < 3; ++f)
@@ -420,9 +503,9 @@ int setup32(mcv_handle *h) {
   HIP_TRY(hipMemcpyAsync(h->join[2], h->lvv[0], np * sizeof(double), hipMemcpyDeviceToDevice,
                          h->stream));
   hipLaunchKernelGGL(band_copy_kernel, dim3((threads + 255) / 256), dim3(256), 0, h->stream,
-                     h->mesh, h->lpu[0], h->lvv[0], h->band_raw);
+                     h->mesh, h->lpu[0], h->lvv[0], h->band_raw[0]);
   HIP_TRY(hipGetLastError());
-  if ((rc = boundary(h, 0))) return rc;
+  if ((rc = boundary(h, BoundaryArgs{h->lpu[0], h->lvv[0], h->band_raw[0]}))) return rc;
   if ((rc = dev_alloc(h, &h->phi_ref, np))) return rc;
   hipLaunchKernelGGL(unpack_pairs_kernel, dim3(1024), dim3(256), 0, h->stream, np, h->lpu[0],
                      h->phi_ref, nullptr);
@@ -440,9 +523,6 @@ int setup32(mcv_handle *h) {
   for (int l = 0; l < 3; ++l)
     if ((rc = dev_alloc_t(h, &h->l32[l], np))) return rc;
   if ((rc = dev_alloc_t(h, &h->c32, np)) || (rc = dev_alloc_t(h, &h->a32, np))) return rc;
-  if ((rc = dev_alloc_t(h, &h->band32, nband / 3)) ||
-      (rc = dev_alloc_t(h, &h->band32c, nband / 3)))
-    return rc;
   double *pgref;
   if ((rc = dev_alloc_t(h, &pgref, np))) return rc;
   hipLaunchKernelGGL(pgref_kernel, dim3(1024), dim3(256), 0, h->stream, h->mesh, h->phi_ref,
@@ -463,17 +543,16 @@ int setup32(mcv_handle *h) {
   m.rdx = 1.0 / d.dx;
   m.r2dx = 1.0 / (2.0 * d.dx);
   m.rdxx = 1.0 / (d.dx * d.dx);
-  m.dxf = d.dx;
+  m.dx = d.dx;
   m.metric_pstride = d.metric_pstride;
-  m.sg = d.sqrtG;
-  m.rsg = d.rsqrtG;
-  m.ig11 = d.ig11;
-  m.ig12 = d.ig12;
-  m.ig22 = d.ig22;
   m.mpack = d.mpack;
-  m.spack = d.spack;
   m.pgref = pgref;
   m.fdE = fdE;
+  m.p2sp = d.p2sp;
+  m.sp2p_ghost = d.sp2p_ghost;
+  m.sp2p_edge = d.sp2p_edge;
+  m.gcoef = d.gcoef;
+  m.giref = d.giref;
   HIP_TRY(hipStreamSynchronize(h->stream));
   return MCV_OK;
 }
@@ -551,8 +630,6 @@ int init_impl(const mcv_config *cfg, const mcv_mesh *mesh, const mcv_state *st,
   m.dv.dx = make_recip(cfg->dx);
   m.dv.dx2 = make_recip(2.0 * cfg->dx);
   m.dv.dxx = make_recip(cfg->dx * cfg->dx);
-  std::vector<double> rsg(np);
-  for (long long g = 0; g < np; ++g) rsg[g] = 1.0 / mesh->sqrtG[g];
   const bool metric_inv = panel_invariant(mesh->sqrtG, per) && panel_invariant(ig11.data(), per) &&
                           panel_invariant(ig12.data(), per) && panel_invariant(ig22.data(), per);
   const long long mcount = metric_inv ? per : np;
@@ -562,8 +639,6 @@ int init_impl(const mcv_config *cfg, const mcv_mesh *mesh, const mcv_state *st,
   double *d;
   if ((rc = upload(h, &d, mesh->sqrtG, mcount))) return rc;
   m.sqrtG = d;
-  if ((rc = upload(h, &d, rsg.data(), mcount))) return rc;
-  m.rsqrtG = d;
   if ((rc = upload(h, &d, ig11.data(), mcount))) return rc;
   m.ig11 = d;
   if ((rc = upload(h, &d, ig12.data(), mcount))) return rc;
@@ -571,19 +646,15 @@ int init_impl(const mcv_config *cfg, const mcv_mesh *mesh, const mcv_state *st,
   if ((rc = upload(h, &d, ig22.data(), mcount))) return rc;
   m.ig22 = d;
   {
-    std::vector<double> mp(4 * mcount), sp(2 * mcount);
+    std::vector<double> mp(4 * mcount);
     for (long long g = 0; g < mcount; ++g) {
       mp[4 * g] = mesh->sqrtG[g];
       mp[4 * g + 1] = ig11[g];
       mp[4 * g + 2] = ig12[g];
       mp[4 * g + 3] = ig22[g];
-      sp[2 * g] = mesh->sqrtG[g];
-      sp[2 * g + 1] = rsg[g];
     }
     if ((rc = upload(h, &d, mp.data(), mp.size()))) return rc;
     m.mpack = reinterpret_cast<const D2 *>(d);
-    if ((rc = upload(h, &d, sp.data(), sp.size()))) return rc;
-    m.spack = reinterpret_cast<const D2 *>(d);
   }
   m.phis_zero = 1;
   for (long long g = 0; g < np && m.phis_zero; ++g) {
@@ -598,22 +669,16 @@ int init_impl(const mcv_config *cfg, const mcv_mesh *mesh, const mcv_state *st,
   if ((rc = upload(h, &d, p2sp.data(), 4 * np))) return rc;
   m.p2sp = d;
   {
-    // line-major matrix tables of the boundary pass (band, ghost and edge points)
+    // line-major matrix tables of the boundary pass (ghost and edge points)
     const int npv = h->npv;
-    std::vector<double> pb(4 * (size_t)6 * 4 * (H + 1) * npv), sg(4 * (size_t)6 * 4 * H * npv),
-        se(4 * (size_t)6 * 4 * npv);
+    std::vector<double> sg(4 * (size_t)6 * 4 * H * npv), se(4 * (size_t)6 * 4 * npv);
     for (int p = 1; p <= 6; ++p)
       for (int side = 0; side < 4; ++side)
         for (int al = 1; al <= npv; ++al) {
-          for (int dd = 1; dd <= H + 1; ++dd) {
-            int i, j;
-            band_ij(npv, side, dd, al, i, j);
-            std::memcpy(&pb[4 * (size_t)band_point(npv, H, p, side, dd, al)],
-                        &p2sp[4 * pidx(h->nh, H, p, i, j)], 4 * sizeof(double));
-            if (dd == 1)
-              std::memcpy(&se[4 * (size_t)edge_point(npv, p, side, al)],
-                          &sp2p[4 * pidx(h->nh, H, p, i, j)], 4 * sizeof(double));
-          }
+          int i, j;
+          band_ij(npv, side, 1, al, i, j);
+          std::memcpy(&se[4 * (size_t)edge_point(npv, p, side, al)],
+                      &sp2p[4 * pidx(h->nh, H, p, i, j)], 4 * sizeof(double));
           for (int k = 1; k <= H; ++k) {
             int hi, hj;
             if (side == 0) { hi = 1 - k; hj = al; }
@@ -624,8 +689,6 @@ int init_impl(const mcv_config *cfg, const mcv_mesh *mesh, const mcv_state *st,
                         &sp2p[4 * pidx(h->nh, H, p, hi, hj)], 4 * sizeof(double));
           }
         }
-    if ((rc = upload(h, &d, pb.data(), pb.size()))) return rc;
-    m.p2sp_band = d;
     if ((rc = upload(h, &d, sg.data(), sg.size()))) return rc;
     m.sp2p_ghost = d;
     if ((rc = upload(h, &d, se.data(), se.size()))) return rc;
@@ -655,7 +718,8 @@ int init_impl(const mcv_config *cfg, const mcv_mesh *mesh, const mcv_state *st,
     if ((rc = dev_alloc(h, &h->acc[0], 2 * np))) return rc;
     if ((rc = dev_alloc(h, &h->acc[2], np))) return rc;
   }
-  if ((rc = dev_alloc(h, &h->band_raw, band_values(cfg->dof, h->npv)))) return rc;
+  for (int b = 0; b < band_count(cfg->scheme); ++b)
+    if ((rc = dev_alloc_t(h, &h->band_raw[b], band_points(cfg->dof, h->npv)))) return rc;
   {
     std::vector<D2> pu(np);
     for (long long g = 0; g < np; ++g) pu[g] = D2{st->phi[g], st->u[g]};
@@ -765,12 +829,7 @@ int mcv_hip_step(mcv_handle *h, int32_t nsteps) {
   if (!h) return fail(MCV_EINVAL, "handle is NULL");
   if (nsteps < 0) return fail(MCV_EINVAL, "nsteps must be >= 0, got %d", nsteps);
   HIP_TRY(hipSetDevice(h->cfg.device));
-  for (int32_t s = 0; s < nsteps; ++s) {
-    int rc = one_step(h);
-    if (rc) return rc;
-    ++h->steps;
-  }
-  return MCV_OK;
+  return run_steps(h, nsteps);
 }
 
 int mcv_hip_sync(mcv_handle *h, mcv_state *out, double *mass, double *energy) {
@@ -895,7 +954,7 @@ int mcv_hip_tendency(mcv_handle *h, const mcv_state *in, double *t_phiG, double 
   a.in_pu = reinterpret_cast<const D2 *>(tin); a.in_v = h->pack[3];
   a.cu0 = h->pack[4]; a.cv0 = h->pack[5];
   a.o_pu = reinterpret_cast<D2 *>(tpu); a.o_v = tv;
-  if ((rc = stage(h, kTend, a))) return rc;
+  if ((rc = stage(h, kTend, a, false))) return rc;
   std::vector<D2> tk(nt);
   HIP_TRY(hipMemcpyAsync(tk.data(), tpu, nt * sizeof(D2), hipMemcpyDeviceToHost, h->stream));
   HIP_TRY(hipMemcpyAsync(t_v, tv, nt * sizeof(double), hipMemcpyDeviceToHost, h->stream));
@@ -953,7 +1012,7 @@ int mcv_hip_tendency_noalloc(mcv_handle *h, const mcv_state *in, double *t_phiG,
   a.in_pu = s_in; a.in_v = h->pack[3];
   a.cu0 = h->pack[4]; a.cv0 = h->pack[5];
   a.o_pu = s_pu; a.o_v = s_v;
-  int rc = stage(h, kTend, a);
+  int rc = stage(h, kTend, a, false);
   if (rc) return rc;
   hipLaunchKernelGGL(unpack_pairs_kernel, dim3(1024), dim3(256), 0, h->stream, nt, s_pu,
                      h->pack[0], h->pack[1]);
@@ -973,11 +1032,7 @@ int mcv_hip_step_timed(mcv_handle *h, int32_t nsteps, double *stage_ms, double *
   HIP_TRY(hipStreamSynchronize(h->stream));
   h->timing = true;
   h->stage_ms = h->boundary_ms = 0.0;
-  int rc = MCV_OK;
-  for (int32_t s = 0; s < nsteps && rc == MCV_OK; ++s) {
-    rc = one_step(h);
-    if (rc == MCV_OK) ++h->steps;
-  }
+  const int rc = run_steps(h, nsteps);
   h->timing = false;
   if (rc) return rc;
   if (stage_ms) *stage_ms = h->stage_ms;
@@ -998,12 +1053,13 @@ int mcv_hip_autotune(mcv_handle *h, int32_t reps, int32_t *tile, double *ms_per_
   a.b_pu = h->lpu[0]; a.b_v = h->lvv[0];
   a.acc_pu = reinterpret_cast<D2 *>(h->acc[0]); a.acc_v = h->acc[2];
   a.o_pu = h->lpu[1]; a.o_v = h->lvv[1];
-  a.band_raw = h->band_raw;
+  a.band_raw = h->band_raw[0];
   if (h->first_pending) { a.cu0 = h->cu0; a.cv0 = h->cv0; }
   a.c1 = 0.5 * h->cfg.dt;
   const int kind = h->cfg.scheme == MCV_RK4 ? kRK4S2 : kRK3S2;
-  const StageArgs32 a32 = h->fp32c ? stage_args32(h, 0, 1, 0.5 * h->cfg.dt) : StageArgs32{};
-  auto run = [&]() { return h->fp32c ? stage32(h, kind, a32) : stage(h, kind, a); };
+  StageArgs32 a32 = h->fp32c ? stage_args32(h, 0) : StageArgs32{};
+  a32.c1 = 0.5 * h->cfg.dt;
+  auto run = [&]() { return h->fp32c ? stage32(h, kind, a32, false) : stage(h, kind, a, false); };
   const int keep = h->tile;
   int best = keep;
   double best_ms = 1e300;

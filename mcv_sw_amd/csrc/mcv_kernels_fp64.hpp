@@ -1,17 +1,19 @@
 // FP64 kernels of the MCV step on gfx950.
 //
-// One RK stage is two launches:
+// One RK stage is one or two launches:
 //   stage_kernel     per (panel, tile): stage the tile and its one-cell halo
 //                    of (phi, u, v) in LDS with the derived E, phiG, contra
 //                    winds; Riemann derivatives at cell ends; interior
 //                    derivatives; tendencies; RK update.  Writes the raw
-//                    updated interior and the band (a raw copy of the H+1
-//                    lines nearest each panel side).
+//                    updated interior and the band (the H+1 lines nearest each
+//                    panel side, winds on the sphere).
 //   boundary_kernel  one item per ghost point, cube-edge point or cube
 //                    vertex: ghost interpolation into the halo and edge/vertex
 //                    averaging (the reference's correct_bdy_ghost), reading
 //                    the band so that no thread reads a point another thread
 //                    rewrites.
+// Small solves take stage_kernel_raw between two stages, whose tiles at the
+// panel sides run the boundary pass on the points they stage.
 // phiG is never stored: every state keeps phiG = phi*sqrtG exactly
 // (time_scheme_mod.F90:85), so it is recomputed from phi where needed.
 #pragma once
@@ -21,117 +23,20 @@
 
 namespace mcv {
 
-// Work item t of correct_bdy_ghost on one level, t in [0, boundary_items()):
-// one ghost point, one edge point or one cube vertex per item.  Every value is
-// read from the band (the raw lines the stage kernel wrote) and the
-// line-major matrix tables, contiguously along the lines; the items are
-// independent, each a short chain of loads.
 template <int DOF>
-__device__ __forceinline__ void boundary_item(const MeshDev &m, const BoundaryArgs &a,
-                                              const int t) {
-  constexpr int H = DOF - 1;
-  const int npv = m.npv, nh = m.nh;
-  const double dx = m.dx;
-  const int nghost = 6 * 4 * H * npv, nedge = 12 * npv;
-  if (t < nghost) {
-    // (panel, side, depth k, along-edge s), s fastest
-    const int s = t % npv + 1, r = t / npv, k = r % H + 1, ps = r / H;
-    const int side = ps % 4, p = ps / 4 + 1;
-    const HaloSrc hs = kHalo[p - 1][side];
-    // Ghost point at depth k (ghost_mod.f90:154-227): the neighbour's line at
-    // normal index k+1 (or nPV-k) is band depth k+1 of the side it is parallel
-    // to; sphere winds through P2SP there and back through SP2P at the ghost
-    // point (spatial_operators_mod.F90:408-492).
-    const int src = hs.col ? (hs.far ? 1 : 0) : (hs.far ? 3 : 2);
-    const int c = m.giref[(k - 1) * npv + (s - 1)];
-    const double cf = m.gcoef[(k - 1) * npv + (s - 1)];
-    double qp[DOF], qz[DOF], qm[DOF];
-#pragma unroll
-    for (int l = 0; l < DOF; ++l) {
-      const int tpos = (c - 1) * H + 1 + l;
-      const int al = hs.rev ? npv + 1 - tpos : tpos;
-      const double ph = ldg(a.band_raw, band_slot(npv, H, hs.q, src, k + 1, 0, al));
-      const double u = ldg(a.band_raw, band_slot(npv, H, hs.q, src, k + 1, 1, al));
-      const double v = ldg(a.band_raw, band_slot(npv, H, hs.q, src, k + 1, 2, al));
-      qp[l] = ph;
-      apply2(m.p2sp_band + 4 * band_point(npv, H, hs.q, src, k + 1, al), u, v, qz[l], qm[l]);
-    }
-    int hi, hj;
-    if (side == 0) { hi = 1 - k; hj = s; }
-    else if (side == 1) { hi = npv + k; hj = s; }
-    else if (side == 2) { hi = s; hj = 1 - k; }
-    else { hi = s; hj = npv + k; }
-    const long long g = pidx(nh, H, p, hi, hj);
-    const double zh = ghost_interp<DOF>(qz, cf, dx), mh = ghost_interp<DOF>(qm, cf, dx);
-    const double ph = ghost_interp<DOF>(qp, cf, dx);
-    double uh, vh;
-    apply2(m.sp2p_ghost + 4 * ghost_point(npv, H, p, side, k, s), zh, mh, uh, vh);
-    a.pu[g] = D2{ph, uh};
-    a.v[g] = vh;
-  } else if (t < nghost + nedge) {
-    // Edge averaging (spatial_operators_mod.F90:298-345), vertices excluded.
-    const int s = (t - nghost) % npv + 1, e = (t - nghost) / npv;
-    if (s > 1 && s < npv) {
-      const EdgePair ep = kEdges[e];
-      const int sb = ep.rev ? npv + 1 - s : s;
-      const double pa = ldg(a.band_raw, band_slot(npv, H, ep.pa, ep.sa, 1, 0, s));
-      const double ua = ldg(a.band_raw, band_slot(npv, H, ep.pa, ep.sa, 1, 1, s));
-      const double va = ldg(a.band_raw, band_slot(npv, H, ep.pa, ep.sa, 1, 2, s));
-      const double pb = ldg(a.band_raw, band_slot(npv, H, ep.pb, ep.sb, 1, 0, sb));
-      const double ub = ldg(a.band_raw, band_slot(npv, H, ep.pb, ep.sb, 1, 1, sb));
-      const double vb = ldg(a.band_raw, band_slot(npv, H, ep.pb, ep.sb, 1, 2, sb));
-      const uint32_t ba = band_point(npv, H, ep.pa, ep.sa, 1, s);
-      const uint32_t bb = band_point(npv, H, ep.pb, ep.sb, 1, sb);
-      int ia, ja, ib, jb;
-      edge_ij(npv, ep.sa, s, ia, ja);
-      edge_ij(npv, ep.sb, sb, ib, jb);
-      const long long ga = pidx(nh, H, ep.pa, ia, ja), gb = pidx(nh, H, ep.pb, ib, jb);
-      double za, ma, zb, mb;
-      apply2(m.p2sp_band + 4 * ba, ua, va, za, ma);
-      apply2(m.p2sp_band + 4 * bb, ub, vb, zb, mb);
-      const double ph = 0.5 * (pa + pb), zu = 0.5 * (za + zb), mu = 0.5 * (ma + mb);
-      double u1, v1, u2, v2;
-      apply2(m.sp2p_edge + 4 * edge_point(npv, ep.pa, ep.sa, s), zu, mu, u1, v1);
-      apply2(m.sp2p_edge + 4 * edge_point(npv, ep.pb, ep.sb, sb), zu, mu, u2, v2);
-      a.pu[ga] = D2{ph, u1}; a.v[ga] = v1;
-      a.pu[gb] = D2{ph, u2}; a.v[gb] = v2;
-    }
-  } else {
-    // Cube vertices (spatial_operators_mod.F90:347-386), reference summation order.
-    const int vx = t - nghost - nedge;
-    double ph[3], z[3], mr[3];
-    long long gg[3];
-    uint32_t eg[3];
-#pragma unroll
-    for (int l = 0; l < 3; ++l) {
-      const VtxPt vp = kVerts[vx][l];
-      const int i = vp.ci ? npv : 1, j = vp.cj ? npv : 1;
-      const int side = vp.ci ? 1 : 0;  // either edge through the corner holds its raw value
-      ph[l] = ldg(a.band_raw, band_slot(npv, H, vp.p, side, 1, 0, j));
-      const double u = ldg(a.band_raw, band_slot(npv, H, vp.p, side, 1, 1, j));
-      const double v = ldg(a.band_raw, band_slot(npv, H, vp.p, side, 1, 2, j));
-      gg[l] = pidx(nh, H, vp.p, i, j);
-      eg[l] = edge_point(npv, vp.p, side, j);
-      apply2(m.p2sp_band + 4 * band_point(npv, H, vp.p, side, 1, j), u, v, z[l], mr[l]);
-    }
-    const double pv = (ph[0] + ph[1] + ph[2]) / 3.0;
-    const double zv = (z[0] + z[1] + z[2]) / 3.0;
-    const double mv = (mr[0] + mr[1] + mr[2]) / 3.0;
-#pragma unroll
-    for (int l = 0; l < 3; ++l) {
-      double u, v;
-      apply2(m.sp2p_edge + 4 * eg[l], zv, mv, u, v);
-      a.pu[gg[l]] = D2{pv, u};
-      a.v[gg[l]] = v;
-    }
-  }
+__device__ __forceinline__ void boundary_item_f64(const MeshDev &m, const BoundaryArgs &a,
+                                                  const int t) {
+  boundary_item<DOF>(m, a.band_raw, t, [&](long long g, const D3 &x) {
+    write_global((MCV_GLOBAL char *)(a.pu + g), D2{x.a, x.b});
+    write_global((MCV_GLOBAL char *)(a.v + g), x.c);
+  });
 }
 
 template <int DOF>
 __global__ __launch_bounds__(256) void boundary_kernel(MeshDev m, BoundaryArgs a) {
   const int nitems = boundary_items(DOF, m.npv);
   for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < nitems; t += gridDim.x * blockDim.x)
-    boundary_item<DOF>(m, a, t);
+    boundary_item_f64<DOF>(m, a, t);
 }
 
 // Reference-layout copy-out of one level: phi, phiG = phi*sqrtG, u, v and

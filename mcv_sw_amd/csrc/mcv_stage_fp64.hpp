@@ -7,14 +7,15 @@
 // cell end of the tile once (the reference computes each interface twice, from
 // both cells).  Phase 2 forms the
 // interior-point derivatives, the vorticity/Coriolis tendencies and the RK
-// update, and writes the raw updated interior plus a raw copy of the H+1
-// lines nearest each panel side (the band) for the boundary pass.  Every loop runs over compile-time
+// update, and writes the raw updated interior plus the band (the H+1 lines
+// nearest each panel side, winds on the sphere) for the boundary pass.  Every loop runs over compile-time
 // extents, so no index needs a run-time integer division.
 #pragma once
 
 #include <type_traits>
 
 #include "mcv_device.hpp"
+#include "mcv_halo.hpp"
 
 namespace mcv {
 
@@ -61,12 +62,68 @@ struct TileLayout {
   }
 };
 
-// One (panel p, tile tx, ty) of the spatial operator + RK stage `kind`.  The
-// caller passes LDS of at least TileLayout<double, DOF, CX, CY>::kBytes and
-// synchronises before reusing it.
+// The waves per SIMD (= workgroups per CU) a stage kernel is compiled for: what
+// the tile's LDS allows, and no more than the words its threads hold leave room
+// for: phase 0 keeps the loads of all a thread's staged points (2 to 4) in
+// registers.  Left to itself the compiler spends registers freely on the
+// boundary pass, which only the tiles at the panel sides enter (5x5 cells MCV4
+// FP64 105 VGPRs instead of 71, FP32C 83 to 105 instead of 55 to 64).
+template <typename T, int DOF, int CX, int CY>
+constexpr int stage_waves() {
+  using TL = TileLayout<T, DOF, CX, CY>;
+  constexpr int lds = (int)(160 * 1024 / TL::kBytes);
+  constexpr int per_thread = (TL::kPts + kStageThreads - 1) / kStageThreads;
+  constexpr int two = sizeof(T) == 8 ? 6 : 8;
+  constexpr int regs = per_thread <= 2 ? two : per_thread == 3 ? (sizeof(T) == 8 ? 4 : 5) : 4;
+  return lds < regs ? lds : regs;
+}
+
+// The boundary pass on the points that the tile stages, where the tile is in
+// reach of a panel side, into the LDS slots that stage_points takes them from;
+// true if there are any.  Only the owner of a point writes it back (to a level
+// that is read again), and every tile takes these points from the band, so no
+// workgroup reads what another writes.
 template <int DOF, int CX, int CY>
-__device__ __forceinline__ void stage_tile(const MeshDev &m, const StageArgs &a, const int kind,
-                                           const int p, const int tx, const int ty, char *smem) {
+__device__ __forceinline__ bool finish_side_points(const MeshDev &m, const StageArgs &a,
+                                                   const int p, const int tx, const int ty,
+                                                   char *smem) {
+  using TL = TileLayout<double, DOF, CX, CY>;
+  constexpr int H = DOF - 1;
+  constexpr int TX = TL::TX, L = TL::TX > TL::TY ? TL::TX : TL::TY;
+  const int npv = m.npv, nh = m.nh, N = m.n;
+  const int cx0 = tx * CX, cy0 = ty * CY;
+  const int ncx = min(CX, N - cx0), ncy = min(CY, N - cy0);
+  const int i0 = cx0 * H + 1, j0 = cy0 * H + 1;
+  const int nx = ncx * H + 1, ny = ncy * H + 1;
+  const TileSides ts = tile_sides(i0, j0, nx + 2 * H, ny + 2 * H, H, npv);
+  if (__builtin_expect(ts.n == 0, 1)) return false;
+  const int TXo = ncx * H + (cx0 + ncx == N ? 1 : 0);
+  const int TYo = ncy * H + (cy0 + ncy == N ? 1 : 0);
+  const uint32_t pbase = (uint32_t)(p - 1) * (uint32_t)(nh * nh);
+  const TL lds(smem);
+  double *const sU = lds.sU, *const sV = lds.sV, *const sPG = lds.sPG;
+  finish_tile<DOF, L>(m, a.band_in, ts, p, i0, j0, nx, ny, [&](int lx, int ly, const D3 &x) {
+    const int li = ly * TX + lx, ox = lx - H, oy = ly - H;
+    sPG[li] = x.a;
+    sU[li] = x.b;
+    sV[li] = x.c;
+    if (a.fin_pu && ox >= 0 && ox < TXo && oy >= 0 && oy < TYo) {
+      const uint32_t g = pbase + mul24(j0 - 1 + ly, nh) + (uint32_t)(i0 - 1 + lx);
+      stg(a.fin_pu, g, D2{x.a, x.b});
+      stg(a.fin_v, g, x.c);
+    }
+  });
+  __syncthreads();
+  return true;
+}
+
+// One (panel p, tile tx, ty) of the spatial operator + RK stage `kind`.
+// `at_side`: finish_side_points has left points in LDS; `winds`: the handed-over
+// contravariant winds are read.
+template <int DOF, int CX, int CY>
+__device__ __forceinline__ void stage_body(const MeshDev &m, const StageArgs &a, const int kind,
+                                           const bool at_side, const bool winds, const int p,
+                                           const int tx, const int ty, char *smem) {
   using TL = TileLayout<double, DOF, CX, CY>;
   constexpr int H = DOF - 1;
   constexpr int NX = TL::NX, NY = TL::NY, TX = TL::TX;
@@ -94,74 +151,92 @@ __device__ __forceinline__ void stage_tile(const MeshDev &m, const StageArgs &a,
   const uint32_t sbase = (uint32_t)(p - 1) * (uint32_t)m.phis_pstride;
   const D2 *const mpk = m.mpack + 2 * (size_t)mbase;  // this panel's packed metric terms
 
+  // the points that finish_side_points has left in LDS: ghost points and edge lines
+  auto finished = [&](int lx, int ly) {
+    const int i = i0 - H + lx, j = j0 - H + ly;
+    return i <= 1 || i >= npv || j <= 1 || j >= npv;
+  };
+
   // Phase 0: stage the cross-shaped tile + halo; derived fields per point.
   // Every thread first issues the loads of all its points, then derives and
   // stores, so that its loads are in flight together.
-  constexpr int kP0 = (TX * TY + kStageThreads - 1) / kStageThreads;
-  for (int t0 = threadIdx.x; t0 < TX * TY; t0 += kP0 * blockDim.x) {
-    double rphi[kP0], ru[kP0], rv[kP0], rsg[kP0], r11[kP0], r12[kP0], r22[kP0], rps[kP0];
-    double rcu[kP0], rcv[kP0];
-    bool live[kP0];
+  // Tiles without such points have a copy of the loop without the test.
+  auto stage_points = [&](auto at_side) {
+    constexpr bool edge = decltype(at_side)::value;
+    constexpr int kP0 = (TX * TY + kStageThreads - 1) / kStageThreads;
+    for (int t0 = threadIdx.x; t0 < TX * TY; t0 += kP0 * blockDim.x) {
+      double rphi[kP0], ru[kP0], rv[kP0], rsg[kP0], r11[kP0], r12[kP0], r22[kP0], rps[kP0];
+      double rcu[kP0], rcv[kP0];
+      bool live[kP0];
 #pragma unroll
-    for (int q = 0; q < kP0; ++q) {
-      const int t = t0 + q * blockDim.x;
-      const int ly = div_small<TX>(t), lx = t - ly * TX;
-      const bool inx = lx >= H && lx < H + nx, iny = ly >= H && ly < H + ny;
-      // outside the tile, or a halo corner (never read)
-      live[q] = t < TX * TY && lx < lw && ly < lh && (inx || iny);
-      if (!live[q]) continue;
-      const uint32_t off = mul24(j0 - 1 + ly, nh) + (uint32_t)(i0 - 1 + lx);
-      const uint32_t g = pbase + off;
-      const D2 pu = ldg(a.in_pu, g);
-      rphi[q] = pu.a;
-      ru[q] = pu.b;
-      rv[q] = ldg(a.in_v, g);
-      const D2 ga = ldg(mpk, 2 * off), gb = ldg(mpk, 2 * off + 1);
-      rsg[q] = ga.a;
-      r11[q] = ga.b;
-      r12[q] = gb.a;
-      r22[q] = gb.b;
-      rps[q] = m.phis_zero ? 0.0 : ldg(m.phi_s, sbase + off);
-      if (a.cu0) {
-        rcu[q] = ldg(a.cu0, g);
-        rcv[q] = ldg(a.cv0, g);
+      for (int q = 0; q < kP0; ++q) {
+        const int t = t0 + q * blockDim.x;
+        const int ly = div_small<TX>(t), lx = t - ly * TX;
+        const bool inx = lx >= H && lx < H + nx, iny = ly >= H && ly < H + ny;
+        // outside the tile, or a halo corner (never read)
+        live[q] = t < TX * TY && lx < lw && ly < lh && (inx || iny);
+        if (!live[q]) continue;
+        const uint32_t off = mul24(j0 - 1 + ly, nh) + (uint32_t)(i0 - 1 + lx);
+        const uint32_t g = pbase + off;
+        if (edge && finished(lx, ly)) {
+          rphi[q] = sPG[t];
+          ru[q] = sU[t];
+          rv[q] = sV[t];
+        } else {
+          const D2 pu = ldg(a.in_pu, g);
+          rphi[q] = pu.a;
+          ru[q] = pu.b;
+          rv[q] = ldg(a.in_v, g);
+        }
+        const D2 ga = ldg(mpk, 2 * off), gb = ldg(mpk, 2 * off + 1);
+        rsg[q] = ga.a;
+        r11[q] = ga.b;
+        r12[q] = gb.a;
+        r22[q] = gb.b;
+        rps[q] = m.phis_zero ? 0.0 : ldg(m.phi_s, sbase + off);
+        if (!edge && winds) {  // handed over with a finished level
+          rcu[q] = ldg(a.cu0, g);
+          rcv[q] = ldg(a.cv0, g);
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < kP0; ++q) {
+        if (!live[q]) continue;
+        const int li = t0 + q * blockDim.x;  // = ly * TX + lx
+        const int ly = div_small<TX>(li), lx = li - ly * TX;
+        const double phi = rphi[q], u = ru[q], v = rv[q], g11 = r11[q], g12 = r12[q],
+                     g22 = r22[q];
+        double cu, cv;
+        if (!edge && winds) {
+          cu = rcu[q];
+          cv = rcv[q];
+        } else {  // cov2contrav (projection_mod.F90:138-148)
+          cu = g11 * u + g12 * v;
+          cv = g12 * u + g22 * v;
+        }
+        const double K = 0.5 * (cu * u + cv * v);  // spatial_operators_mod.F90:60-61
+        sE[li] = phi + rps[q] + K;
+        sU[li] = u;
+        sV[li] = v;
+        sPG[li] = phi * rsg[q];
+        const bool inx = lx >= H && lx < H + nx, iny = ly >= H && ly < H + ny;
+        if (iny) sCU[TL::cu_at(lx, ly)] = cu;
+        if (inx) sCV[TL::cv_at(lx, ly)] = cv;
+        if (inx && iny) {
+          const int ox = lx - H, oy = ly - H;
+          lds.sSG[TL::core_at(lx, ly)] = rsg[q];
+          // the wave speed's square root is left to phase 1, whose lanes are all
+          // cell ends (one per thread there; here four, with most lanes idle:
+          // MCV4 6x96^2 90.7 -> 88.9 us, 6x384^2 1078 -> 1070 us per RK4 step)
+          const int cx = div_small<H>(ox), cy = div_small<H>(oy);
+          if (ox == cx * H) lamx[cx * NY + oy] = g11 * phi;
+          if (oy == cy * H) lamy[cy * NX + ox] = g22 * phi;
+        }
       }
     }
-#pragma unroll
-    for (int q = 0; q < kP0; ++q) {
-      if (!live[q]) continue;
-      const int li = t0 + q * blockDim.x;  // = ly * TX + lx
-      const int ly = div_small<TX>(li), lx = li - ly * TX;
-      const double phi = rphi[q], u = ru[q], v = rv[q], g11 = r11[q], g12 = r12[q],
-                   g22 = r22[q];
-      double cu, cv;
-      if (a.cu0) {
-        cu = rcu[q];
-        cv = rcv[q];
-      } else {  // cov2contrav (projection_mod.F90:138-148)
-        cu = g11 * u + g12 * v;
-        cv = g12 * u + g22 * v;
-      }
-      const double K = 0.5 * (cu * u + cv * v);  // spatial_operators_mod.F90:60-61
-      sE[li] = phi + rps[q] + K;
-      sU[li] = u;
-      sV[li] = v;
-      sPG[li] = phi * rsg[q];
-      const bool inx = lx >= H && lx < H + nx, iny = ly >= H && ly < H + ny;
-      if (iny) sCU[TL::cu_at(lx, ly)] = cu;
-      if (inx) sCV[TL::cv_at(lx, ly)] = cv;
-      if (inx && iny) {
-        const int ox = lx - H, oy = ly - H;
-        lds.sSG[TL::core_at(lx, ly)] = rsg[q];
-        // the wave speed's square root is left to phase 1, whose lanes are all
-        // cell ends (one per thread there; here four, with most lanes idle:
-        // MCV4 6x96^2 90.7 -> 88.9 us, 6x384^2 1078 -> 1070 us per RK4 step)
-        const int cx = div_small<H>(ox), cy = div_small<H>(oy);
-        if (ox == cx * H) lamx[cx * NY + oy] = g11 * phi;
-        if (oy == cy * H) lamy[cy * NX + ox] = g22 * phi;
-      }
-    }
-  }
+  };
+  if (at_side) stage_points(std::true_type{});
+  else stage_points(std::false_type{});
   __syncthreads();
 
   // Phase 1: Riemann derivatives at every cell end of the core, x then y.  The
@@ -390,30 +465,71 @@ __device__ __forceinline__ void stage_tile(const MeshDev &m, const StageArgs &a,
         stg(a.o_pu, g, D2{phi, u});
         stg(a.o_v, g, v);
         // raw copy of the lines nearest each side for the boundary pass
-        if (i <= H + 1 || i >= npv - H || j <= H + 1 || j >= npv - H) {
-          const double vals[3] = {phi, u, v};
-#pragma unroll
-          for (int fl = 0; fl < 3; ++fl) {
-            if (i <= H + 1) stg(a.band_raw, band_slot(npv, H, p, 0, i, fl, j), vals[fl]);
-            if (i >= npv - H) stg(a.band_raw, band_slot(npv, H, p, 1, npv + 1 - i, fl, j), vals[fl]);
-            if (j <= H + 1) stg(a.band_raw, band_slot(npv, H, p, 2, j, fl, i), vals[fl]);
-            if (j >= npv - H) stg(a.band_raw, band_slot(npv, H, p, 3, npv + 1 - j, fl, i), vals[fl]);
-          }
-        }
+        if (i <= H + 1 || i >= npv - H || j <= H + 1 || j >= npv - H)
+          put_band(a.band_raw, npv, H, p, i, j, m.p2sp + 4 * (size_t)g, phi, u, v);
       }
     }
   }
+}
+
+// A stage of one tile.  `raw`: the input is as a stage left it, so the tiles at
+// the panel sides form its halo and edge lines themselves, from that stage's
+// band.  The caller passes LDS of at least TileLayout<double, DOF, CX, CY>::kBytes
+// and synchronises before reusing it.
+template <int DOF, int CX, int CY, bool Reread>
+__device__ __forceinline__ void stage_tile(const MeshDev &m, const StageArgs &a, const int kind,
+                                   const bool raw, const bool winds, const int p, const int tx, const int ty,
+                                   char *smem) {
+  const bool at_side = raw && finish_side_points<DOF, CX, CY>(m, a, p, tx, ty, smem);
+  // Reread: the arguments are loaded again after the boundary pass; kept across
+  // it they overflow the scalar registers (57 spills, 300 instructions, MCV4 5x5)
+  if constexpr (Reread)
+    stage_body<DOF, CX, CY>(reread(m), reread(a), kind, at_side, winds, p, tx, ty, smem);
+  else
+    stage_body<DOF, CX, CY>(m, a, kind, at_side, winds, p, tx, ty, smem);
 }
 
 // Single-solve stage kernel: one workgroup per (panel, tile), blocks of one
 // XCD on neighbouring tiles.
 template <int DOF, int KIND, int CX, int CY>
 __global__ __launch_bounds__(kStageThreads, 6) void stage_kernel(MeshDev m, StageArgs a,
-                                                              int tiles_x) {
+                                                                 int tiles_x) {
   __shared__ __align__(16) char smem[TileLayout<double, DOF, CX, CY>::kBytes];
   const int L = xcd_remap(blockIdx.x, gridDim.x);
   const int tile = L / 6;
-  stage_tile<DOF, CX, CY>(m, a, KIND, L % 6 + 1, tile % tiles_x, tile / tiles_x, smem);
+  stage_body<DOF, CX, CY>(m, a, KIND, false, a.cu0 != nullptr, L % 6 + 1, tile % tiles_x,
+                          tile / tiles_x, smem);
+}
+
+// The same on a raw input.
+template <typename M, typename A>
+struct StageLaunch {
+  M m;
+  A a;
+  int tiles_x;
+};
+
+// The launch's arguments where they are, in the kernel argument segment (the
+// kernel has no others).
+template <typename L>
+__device__ __forceinline__ const L &launch_args(const L &l) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return *(const L *)(const __attribute__((address_space(4))) L *)
+      __builtin_amdgcn_kernarg_segment_ptr();
+#else
+  return l;
+#endif
+}
+
+template <int DOF, int KIND, int CX, int CY>
+__global__ __launch_bounds__(kStageThreads, (stage_waves<double, DOF, CX, CY>())) void
+stage_kernel_raw(StageLaunch<MeshDev, StageArgs> args) {
+  __shared__ __align__(16) char smem[TileLayout<double, DOF, CX, CY>::kBytes];
+  const StageLaunch<MeshDev, StageArgs> &k = launch_args(args);
+  const int L = xcd_remap(blockIdx.x, gridDim.x);
+  const int tile = L / 6, tiles_x = k.tiles_x;
+  stage_tile<DOF, CX, CY, true>(k.m, k.a, KIND, true, false, L % 6 + 1, tile % tiles_x,
+                                tile / tiles_x, smem);
 }
 
 }  // namespace mcv
