@@ -36,6 +36,7 @@
 #include <utility>
 #include <vector>
 
+#define MCV_POINTERS_IN_MEMORY  // see mcv_device.hpp
 #include "../../include/mcv_hip.h"
 #include "mcv_handle.hpp"
 #include "mcv_kernels_fp64.hpp"

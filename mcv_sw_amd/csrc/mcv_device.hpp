@@ -203,10 +203,14 @@ __device__ __forceinline__ int div_small(int t) {
 // byte offset, which the global load/store instructions take directly (no
 // 64-bit address arithmetic per access).  The library keeps every array that
 // the stage kernels touch below 2^32 bytes (n <= 2048).
-// The accesses name the global address space: a pointer that comes out of a
-// struct in memory is generic to the compiler, and a generic (flat) access
-// counts as an LDS access as well, so that every LDS wait would wait for it.
-#if defined(__HIP_DEVICE_COMPILE__)
+// MCV_POINTERS_IN_MEMORY (the batched kernels, whose pointers come out of
+// descriptors in device memory and are generic to the compiler): the accesses
+// name the global address space, since a generic (flat) access counts as an LDS
+// access as well.  The single-solve kernels' pointers are kernel arguments,
+// known to be global; spelled out there too, the loads were scheduled worse
+// (MCV4 6x384^2 per RK4 step: FP64 1025 -> 1047 us, FP32C 717 -> 764; the
+// 20-member ensemble gains, 100.7 -> 99.0 us per stage).
+#if defined(__HIP_DEVICE_COMPILE__) && defined(MCV_POINTERS_IN_MEMORY)
 #define MCV_GLOBAL __attribute__((address_space(1)))
 #else
 #define MCV_GLOBAL
@@ -224,6 +228,9 @@ __device__ __forceinline__ void write_as(MCV_GLOBAL char *p, S v) {
 }
 template <typename T>
 __device__ __forceinline__ T read_global(const MCV_GLOBAL char *p) {
+#ifndef MCV_POINTERS_IN_MEMORY
+  return *reinterpret_cast<const T *>(p);
+#else
   if constexpr (std::is_same_v<T, D2>) {
     const mcv_d2 v = read_as<mcv_d2>(p);
     return D2{v[0], v[1]};
@@ -237,9 +244,13 @@ __device__ __forceinline__ T read_global(const MCV_GLOBAL char *p) {
   } else {
     return read_as<T>(p);
   }
+#endif
 }
 template <typename T>
 __device__ __forceinline__ void write_global(MCV_GLOBAL char *p, const T &v) {
+#ifndef MCV_POINTERS_IN_MEMORY
+  *reinterpret_cast<T *>(p) = v;
+#else
   if constexpr (std::is_same_v<T, D2>) {
     write_as(p, mcv_d2{v.a, v.b});
   } else if constexpr (std::is_same_v<T, D3>) {
@@ -249,6 +260,7 @@ __device__ __forceinline__ void write_global(MCV_GLOBAL char *p, const T &v) {
   } else {
     write_as(p, v);
   }
+#endif
 }
 
 template <typename T>

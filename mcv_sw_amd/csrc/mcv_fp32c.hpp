@@ -489,8 +489,10 @@ __device__ __forceinline__ void stage_body_f32(const MeshF32 &m, const StageArgs
           const double bp = last ? (double)hi.a + (double)lo.a : (double)hi.a;
           const double bu = last ? (double)hi.b + (double)lo.b : (double)hi.b;
           const double bv = last ? (double)hi.c + (double)lo.c : (double)hi.c;
-          const size_t g = pbase + mul24(j + H - 1, nh) + (uint32_t)(i + H - 1);
-          put_band(a.band_raw, npv, H, p, i, j, m.p2sp + 4 * g, bp, bu, bv);
+          const uint32_t g = pbase + mul24(j + H - 1, nh) + (uint32_t)(i + H - 1);
+          const D2 p0 = ldg((const D2 *)m.p2sp, 2 * g), p1 = ldg((const D2 *)m.p2sp, 2 * g + 1);
+          const double P[4] = {p0.a, p0.b, p1.a, p1.b};
+          put_band(a.band_raw, npv, H, p, i, j, P, bp, bu, bv);
         }
       }
     }

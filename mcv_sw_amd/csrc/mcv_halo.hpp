@@ -25,7 +25,9 @@ __device__ __forceinline__ void put_band(D3 *band, const int npv, const int H, c
                                          const double ph, const double u, const double v) {
   D3 r;
   r.a = ph;
-  apply2(P, u, v, r.b, r.c);  // sphere winds (spatial_operators_mod.F90:391-405)
+  // sphere winds (spatial_operators_mod.F90:391-405)
+  r.b = P[0] * u + P[2] * v;
+  r.c = P[1] * u + P[3] * v;
   if (i <= H + 1) stg(band, band_point(npv, H, p, 0, i, j), r);
   if (i >= npv - H) stg(band, band_point(npv, H, p, 1, npv + 1 - i, j), r);
   if (j <= H + 1) stg(band, band_point(npv, H, p, 2, j, i), r);
