@@ -106,6 +106,8 @@ inline hipError_t hipMalloc(void **p, size_t n) {
   return *p ? hipSuccess : 2;
 }
 inline hipError_t hipFree(void *p) { std::free(p); return hipSuccess; }
+inline hipError_t hipHostMalloc(void **p, size_t n, unsigned) { return hipMalloc(p, n); }
+inline hipError_t hipHostFree(void *p) { return hipFree(p); }
 inline hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind) {
   std::memcpy(d, s, n);
   return hipSuccess;

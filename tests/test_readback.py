@@ -1,0 +1,50 @@
+"""Large read-backs through the copy threads against single fields read one at
+a time (plain copies): the same bytes, also with two solves read at once (one
+of them finds the copy threads busy).  Sizes on both sides of the rule: six
+fields of 1.7 MB (four threads) and of 7 MB (eight), none a whole number of
+chunks."""
+import threading
+
+import numpy as np
+import pytest
+
+import cases
+from mcv_sw_amd import capi
+
+
+def _check(lib, dof, n):
+    m = cases.mesh(dof, n)
+    st = cases.case5(m)
+    with capi.Solver(dof, n, 50.0, m, st, lib=lib) as a, capi.Solver(dof, n, 50.0, m, st,
+                                                                     lib=lib) as b:
+        one = {k: a.sync(fields=(k,), integrals=False)[k] for k in capi.STATE_FIELDS}
+        outs = [None, None]
+
+        def read(i, s):
+            outs[i] = [s.sync(integrals=False) for _ in range(3)]
+
+        team = [threading.Thread(target=read, args=x) for x in ((0, a), (1, b))]
+        for t in team:
+            t.start()
+        for t in team:
+            t.join()
+        for out in outs[0] + outs[1]:
+            for k in capi.STATE_FIELDS:
+                assert np.array_equal(out[k], one[k]), k
+
+
+@pytest.mark.parametrize("dof,n", [(4, 60), (3, 190)])
+def test_emulated_large_readback(emu_lib, dof, n):
+    # one solve at a time here: the shim's launches share their LDS statics
+    m = cases.mesh(dof, n)
+    st = cases.case5(m)
+    with capi.Solver(dof, n, 50.0, m, st, lib=emu_lib) as s:
+        out = s.sync(integrals=False)
+        for k in capi.STATE_FIELDS:
+            assert np.array_equal(out[k], s.sync(fields=(k,), integrals=False)[k]), k
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dof,n", [(4, 60), (3, 190)])
+def test_gpu_large_readback(hip_lib, dof, n):
+    _check(None, dof, n)
