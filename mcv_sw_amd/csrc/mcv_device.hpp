@@ -201,8 +201,13 @@ __device__ __forceinline__ int div_small(int t) {
 
 // Element idx of a device array addressed as a uniform base plus a 32-bit
 // byte offset, which the global load/store instructions take directly (no
-// 64-bit address arithmetic per access).  The library keeps every array that
-// the stage kernels touch below 2^32 bytes (n <= 2048).
+// 64-bit address arithmetic per access).  Arrays indexed over all six panels
+// hold up to 16 bytes a point, which stays below 2^32 bytes up to kMaxN; the
+// 32-byte records (mpack, p2sp) do not, so their base is a panel's own.
+constexpr int kMaxN = 2048;  // largest accepted n
+constexpr unsigned long long kMaxPanelPoints = (3ull * kMaxN + 7) * (3 * kMaxN + 7);  // MCV4
+static_assert(6 * kMaxPanelPoints * sizeof(D2) <= 1ull << 32, "16 bytes a point, all panels");
+static_assert(kMaxPanelPoints * 2 * sizeof(D2) <= 1ull << 32, "32 bytes a point, one panel");
 // MCV_POINTERS_IN_MEMORY (the batched kernels, whose pointers come out of
 // descriptors in device memory and are generic to the compiler): the accesses
 // name the global address space, since a generic (flat) access counts as an LDS

@@ -166,10 +166,12 @@ __device__ __forceinline__ void stage_body_f32(const MeshF32 &m, const StageArgs
   const int TXo = ncx * H + (cx0 + ncx == N ? 1 : 0);
   const int TYo = ncy * H + (cy0 + ncy == N ? 1 : 0);
   const int lw = nx + 2 * H, lh = ny + 2 * H;
-  // 32-bit point indices (every array here is below 2^32 bytes)
+  // 32-bit point indices over all panels; the 32-byte records (mpack, p2sp)
+  // are indexed within their panel (see ldg)
   const uint32_t pbase = (uint32_t)(p - 1) * (uint32_t)(nh * nh);
   const uint32_t mbase = (uint32_t)(p - 1) * (uint32_t)m.metric_pstride;
   const D2 *const mpk = m.mpack + 2 * (size_t)mbase;  // this panel's packed metric terms
+  const D2 *const psp = (const D2 *)m.p2sp + 2 * (size_t)pbase;  // and its A*IG
   // byte offset of point (row, col) of this panel in the 12-byte record arrays,
   // from full-rate 24-bit multiplies (row, col < nh <= 6148)
   const uint32_t pb12 = 12u * pbase, nh12 = 12u * (uint32_t)nh;
@@ -489,8 +491,8 @@ __device__ __forceinline__ void stage_body_f32(const MeshF32 &m, const StageArgs
           const double bp = last ? (double)hi.a + (double)lo.a : (double)hi.a;
           const double bu = last ? (double)hi.b + (double)lo.b : (double)hi.b;
           const double bv = last ? (double)hi.c + (double)lo.c : (double)hi.c;
-          const uint32_t g = pbase + mul24(j + H - 1, nh) + (uint32_t)(i + H - 1);
-          const D2 p0 = ldg((const D2 *)m.p2sp, 2 * g), p1 = ldg((const D2 *)m.p2sp, 2 * g + 1);
+          const uint32_t off = mul24(j + H - 1, nh) + (uint32_t)(i + H - 1);
+          const D2 p0 = ldg(psp, 2 * off), p1 = ldg(psp, 2 * off + 1);
           const double P[4] = {p0.a, p0.b, p1.a, p1.b};
           put_band(a.band_raw, npv, H, p, i, j, P, bp, bu, bv);
         }

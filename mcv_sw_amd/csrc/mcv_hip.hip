@@ -336,8 +336,9 @@ int validate(const mcv_config *c) {
   if (c->abi_version != MCV_ABI_VERSION)
     return fail(MCV_EINVAL, "abi_version %d, library is %d", c->abi_version, MCV_ABI_VERSION);
   if (c->dof != 3 && c->dof != 4) return fail(MCV_EINVAL, "dof must be 3 or 4, got %d", c->dof);
-  // every per-point array the stage kernels index stays below 2^32 bytes
-  if (c->n < 2 || c->n > 2048) return fail(MCV_EINVAL, "n must be in [2, 2048], got %d", c->n);
+  // the stage kernels' 32-bit byte offsets reach every point up to kMaxN (see ldg)
+  if (c->n < 2 || c->n > kMaxN)
+    return fail(MCV_EINVAL, "n must be in [2, %d], got %d", kMaxN, c->n);
   if (c->scheme != MCV_RK4 && c->scheme != MCV_RK3_TVD)
     return fail(MCV_EINVAL, "Unknown integral scheme %d, select MCV_RK3_TVD or MCV_RK4",
                 c->scheme);

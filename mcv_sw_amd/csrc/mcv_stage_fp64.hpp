@@ -145,11 +145,13 @@ __device__ __forceinline__ void stage_body(const MeshDev &m, const StageArgs &a,
   const int TXo = ncx * H + (cx0 + ncx == N ? 1 : 0);     // owned points
   const int TYo = ncy * H + (cy0 + ncy == N ? 1 : 0);
   const int lw = nx + 2 * H, lh = ny + 2 * H;
-  // 32-bit point indices (every array here is below 2^32 bytes)
+  // 32-bit point indices over all panels; the 32-byte records (mpack, p2sp)
+  // are indexed within their panel (see ldg)
   const uint32_t pbase = (uint32_t)(p - 1) * (uint32_t)(nh * nh);
   const uint32_t mbase = (uint32_t)(p - 1) * (uint32_t)m.metric_pstride;
   const uint32_t sbase = (uint32_t)(p - 1) * (uint32_t)m.phis_pstride;
   const D2 *const mpk = m.mpack + 2 * (size_t)mbase;  // this panel's packed metric terms
+  const D2 *const psp = (const D2 *)m.p2sp + 2 * (size_t)pbase;  // and its A*IG
 
   // the points that finish_side_points has left in LDS: ghost points and edge lines
   auto finished = [&](int lx, int ly) {
@@ -363,8 +365,8 @@ __device__ __forceinline__ void stage_body(const MeshDev &m, const StageArgs &a,
       const int bi = i0 + ox, bj = j0 + oy;
       near[q] = kind != kTend && (bi <= H + 1 || bi >= npv - H || bj <= H + 1 || bj >= npv - H);
       if (near[q]) {
-        rp0[q] = ldg((const D2 *)m.p2sp, 2 * g);
-        rp1[q] = ldg((const D2 *)m.p2sp, 2 * g + 1);
+        rp0[q] = ldg(psp, 2 * off);
+        rp1[q] = ldg(psp, 2 * off + 1);
       }
       if (need_base) {
         const D2 bpu = ldg(a.b_pu, g);
