@@ -140,11 +140,12 @@ int mcv_hip_step_timed(mcv_handle *h, int32_t nsteps, double *stage_ms,
                        double *boundary_ms);
 
 /* Tile-shape autotuner (no counterpart in the reference): times each of the
- * library's MCV_TILE_VARIANTS stage-kernel tile shapes for this solve (reps
- * launches each, on scratch levels, so the trajectory is not changed), keeps
- * the fastest for later steps and returns its index and, if ms_per_stage is
- * not NULL, the mean milliseconds of every variant (MCV_TILE_VARIANTS
- * doubles).  Blocks. */
+ * library's MCV_TILE_VARIANTS stage-kernel tile shapes for this solve (a stage
+ * as the steps run it, its boundary pass included, in reps rounds over the
+ * shapes, on scratch levels, so the trajectory is not changed), keeps the
+ * fastest for later steps and returns its index and, if ms_per_stage is not
+ * NULL, the milliseconds per stage of every variant in its best round
+ * (MCV_TILE_VARIANTS doubles).  Blocks. */
 #define MCV_TILE_VARIANTS 4
 int mcv_hip_autotune(mcv_handle *h, int32_t reps, int32_t *tile, double *ms_per_stage);
 

@@ -75,15 +75,18 @@ size_t footprint_bytes(const mcv_config *c);
 
 // The RK stages of a time step (time_scheme_mod.F90:13-69).  Levels: 0 = Yn
 // (updated in place by the last stage), 1 and 2 = intermediate stage states.
-// Each stage writes a band of its own and reads the one before it, which other
-// workgroups of the same launch may still be reading: RK4 alternates between
-// two bands, RK3, with its odd number of stages, goes round three.
+// Each stage has a band of its own and reads that of the stage before it, which
+// other workgroups of the same launch may still be reading; the last stage's
+// keeps the raw lines of Y_n until the next step's last stage.
 struct StageSpec {
   int kind, in, out;
   double c1;  // stage increment coefficient (x dt)
 };
 inline int stage_count(int scheme) { return scheme == MCV_RK4 ? 4 : 3; }
-inline int band_count(int scheme) { return scheme == MCV_RK4 ? 2 : 3; }
+// The second stage is the one that the autotuners repeat: S1, S2, the
+// accumulator and the first two bands, all it touches beside reading Y_n, are
+// written anew by every step.
+constexpr int kTuneStage = 1;
 inline StageSpec stage_spec(const mcv_config &c, int s) {
   const double dt = c.dt;
   const StageSpec rk4[4] = {{kRK4S1, 0, 1, 0.5 * dt}, {kRK4S2, 1, 2, 0.5 * dt},
@@ -100,6 +103,36 @@ StageArgs32 stage_args32(const mcv_handle *h, int s);
 BoundaryArgs boundary_args64(const mcv_handle *h, int s);
 BoundaryArgs32 boundary_args32(const mcv_handle *h, int s);
 
+// Milliseconds per stage of every tile shape: use(v) switches to shape v,
+// stage() enqueues a stage as the steps would run it, boundary launch included
+// where the shape needs one.  The shapes take turns, `reps` rounds, so that a
+// drift meets them all; each turn is timed over at least kTuneMs (a stretch of
+// three stages of 7 us told shapes 5% apart wrongly) behind a stage that is not,
+// and the best turn counts.
+constexpr float kTuneMs = 0.25f;
+template <class Use, class Stage>
+int time_shapes(hipStream_t stream, hipEvent_t *ev, int reps, const Use &use, const Stage &stage,
+                double *ms) {
+  int stages[kTileVariants];
+  for (int r = -1; r < reps; ++r)  // the first round sets the stretches (and loads the code)
+    for (int v = 0; v < kTileVariants; ++v) {
+      const int n = r < 0 ? 1 : stages[v];
+      int rc = use(v);
+      for (int k = 0; k <= n && rc == MCV_OK; ++k) {
+        if (k == 1) HIP_TRY(hipEventRecord(ev[0], stream));
+        rc = stage();
+      }
+      if (rc) return rc;
+      HIP_TRY(hipEventRecord(ev[1], stream));
+      HIP_TRY(hipEventSynchronize(ev[1]));
+      float t = 0.f;
+      HIP_TRY(hipEventElapsedTime(&t, ev[0], ev[1]));
+      if (r < 0) stages[v] = t * 16 < kTuneMs ? 16 : 1 + (int)(kTuneMs / t);
+      else if (r == 0 || t / n < ms[v]) ms[v] = t / n;
+    }
+  return MCV_OK;
+}
+
 }  // namespace mcv
 
 // One solve on one device.
@@ -115,7 +148,7 @@ struct mcv_handle {
   double *lvv[3] = {};         //   and v
   double *phi_ref = nullptr;   // FP32C: the projected initial geopotential (FP64)
   double *acc[3] = {};         // RK4 accumulator: acc[0] {phiG, u} pairs, acc[2] v
-  mcv::D3 *band_raw[3] = {};   // raw band lines written by the stage kernel
+  mcv::D3 *band_raw[4] = {};   // raw band lines written by the stage kernel, per stage
   double *cu0 = nullptr, *cv0 = nullptr;  // host contra winds until the first stage
   bool first_pending = true;
   double *partials = nullptr;

@@ -51,7 +51,7 @@ size_t footprint_bytes(const mcv_config *c) {
   const bool fp32c = c->precision == MCV_FP32C;
   b += (fp32c ? 3 : 9) * d(np);                       // FP64 levels
   if (!fp32c) b += 3 * d(np);                          // RK4 accumulator
-  b += band_count(c->scheme) * d(nband) + 2 * d(np) + d(4 * diag_blocks) + d(2) + 6 * d(np);
+  b += stage_count(c->scheme) * d(nband) + 2 * d(np) + d(4 * diag_blocks) + d(2) + 6 * d(np);
   if (fp32c)  // join, phi_ref, phi_ref*sqrtG, FP32 {reference gradient, Coriolis, 0},
               // levels, compensation, accumulator
     b += 3 * d(np) + d(np) + d(np) + 4 * f(np) + 3 * f(3 * np) + f(3 * np) + f(3 * np);
@@ -60,14 +60,14 @@ size_t footprint_bytes(const mcv_config *c) {
 
 StageArgs stage_args64(const mcv_handle *h, int s) {
   const StageSpec sp = stage_spec(h->cfg, s);
-  const int nst = stage_count(h->cfg.scheme), nb = band_count(h->cfg.scheme);
+  const int nst = stage_count(h->cfg.scheme);
   StageArgs a{};
   a.in_pu = h->lpu[sp.in]; a.in_v = h->lvv[sp.in];
   a.b_pu = h->lpu[0]; a.b_v = h->lvv[0];
   a.acc_pu = reinterpret_cast<D2 *>(h->acc[0]); a.acc_v = h->acc[2];
   a.o_pu = h->lpu[sp.out]; a.o_v = h->lvv[sp.out];
-  a.band_raw = h->band_raw[s % nb];
-  a.band_in = h->band_raw[(s + nst - 1) % nst % nb];
+  a.band_raw = h->band_raw[s];
+  a.band_in = h->band_raw[(s + nst - 1) % nst];
   if (s == 0) { a.fin_pu = h->lpu[0]; a.fin_v = h->lvv[0]; }
   a.c1 = sp.c1;
   return a;
@@ -75,12 +75,12 @@ StageArgs stage_args64(const mcv_handle *h, int s) {
 
 BoundaryArgs boundary_args64(const mcv_handle *h, int s) {
   const int out = stage_spec(h->cfg, s).out;
-  return BoundaryArgs{h->lpu[out], h->lvv[out], h->band_raw[s % band_count(h->cfg.scheme)]};
+  return BoundaryArgs{h->lpu[out], h->lvv[out], h->band_raw[s]};
 }
 
 StageArgs32 stage_args32(const mcv_handle *h, int s) {
   const StageSpec sp = stage_spec(h->cfg, s);
-  const int nst = stage_count(h->cfg.scheme), nb = band_count(h->cfg.scheme);
+  const int nst = stage_count(h->cfg.scheme);
   StageArgs32 a{};
   a.in = h->l32[sp.in];
   a.b = h->l32[0];
@@ -88,8 +88,8 @@ StageArgs32 stage_args32(const mcv_handle *h, int s) {
   a.acc = h->a32;
   a.o = h->l32[sp.out];
   if (sp.out == 0) a.oc = h->c32;  // the step's last stage writes Y_n+1 with its compensation
-  a.band_raw = h->band_raw[s % nb];
-  a.band_in = h->band_raw[(s + nst - 1) % nst % nb];
+  a.band_raw = h->band_raw[s];
+  a.band_in = h->band_raw[(s + nst - 1) % nst];
   if (s == 0) {  // Y_n, raw from the step before: base of the stages that follow
     a.fin = h->l32[0];
     a.fin_c = h->c32;
@@ -105,7 +105,7 @@ BoundaryArgs32 boundary_args32(const mcv_handle *h, int s) {
   BoundaryArgs32 b{};
   b.lev = h->l32[out];
   if (out == 0) b.comp = h->c32;  // Y_n carries its compensation words
-  b.band_raw = h->band_raw[s % band_count(h->cfg.scheme)];
+  b.band_raw = h->band_raw[s];
   return b;
 }
 
@@ -546,10 +546,9 @@ int boundary_pass(mcv_handle *h, int s) {
   return MCV_OK;
 }
 
-// nsteps time steps.  Y_n is finished when they are enqueued, as a following
-// call and the read-backs expect it.
-int run_steps(mcv_handle *h, int32_t nsteps) {
-  const int nst = stage_count(h->cfg.scheme), t = h->tile;
+// Whether the boundary pass runs inside the stages at the current tile shape.
+bool fused_sides(const mcv_handle *h) {
+  const int t = h->tile;
   int cx, cy;
   if (h->fp32c) {
     cx = h->cfg.dof == 3 ? TileSet32<3>::cx[t] : TileSet32<4>::cx[t];
@@ -559,7 +558,14 @@ int run_steps(mcv_handle *h, int32_t nsteps) {
     cy = h->cfg.dof == 3 ? TileSet<3>::cy[t] : TileSet<4>::cy[t];
   }
   const int n = h->cfg.n;
-  const bool fused = sides_in_stage(t, 6LL * ((n + cx - 1) / cx) * ((n + cy - 1) / cy));
+  return sides_in_stage(t, 6LL * ((n + cx - 1) / cx) * ((n + cy - 1) / cy));
+}
+
+// nsteps time steps.  Y_n is finished when they are enqueued, as a following
+// call and the read-backs expect it.
+int run_steps(mcv_handle *h, int32_t nsteps) {
+  const int nst = stage_count(h->cfg.scheme);
+  const bool fused = fused_sides(h);
   bool raw = false;  // the next stage's input is as a stage left it
   for (int32_t k = 0; k < nsteps; ++k) {
     for (int s = 0; s < nst; ++s) {
@@ -856,7 +862,7 @@ int init_impl(const mcv_config *cfg, const mcv_mesh *mesh, const mcv_state *st,
     if ((rc = dev_alloc(h, &h->acc[0], 2 * np))) return rc;
     if ((rc = dev_alloc(h, &h->acc[2], np))) return rc;
   }
-  for (int b = 0; b < band_count(cfg->scheme); ++b)
+  for (int b = 0; b < stage_count(cfg->scheme); ++b)
     if ((rc = dev_alloc_t(h, &h->band_raw[b], band_points(cfg->dof, h->npv)))) return rc;
   {
     std::vector<D2> pu(np);
@@ -1184,40 +1190,28 @@ int mcv_hip_autotune(mcv_handle *h, int32_t reps, int32_t *tile, double *ms_per_
   if (reps < 1) return fail(MCV_EINVAL, "reps must be >= 1");
   HIP_TRY(hipSetDevice(h->cfg.device));
   HIP_TRY(hipStreamSynchronize(h->stream));
-  // A representative stage (reads Yn and the accumulator, writes S1 and the
-  // accumulator): S1, the accumulator and the band are rewritten by
-  // the first stage of every step, so timing never changes the trajectory.
-  StageArgs a{};
-  a.in_pu = h->lpu[0]; a.in_v = h->lvv[0];
-  a.b_pu = h->lpu[0]; a.b_v = h->lvv[0];
-  a.acc_pu = reinterpret_cast<D2 *>(h->acc[0]); a.acc_v = h->acc[2];
-  a.o_pu = h->lpu[1]; a.o_v = h->lvv[1];
-  a.band_raw = h->band_raw[0];
-  if (h->first_pending) { a.cu0 = h->cu0; a.cv0 = h->cv0; }
-  a.c1 = 0.5 * h->cfg.dt;
-  const int kind = h->cfg.scheme == MCV_RK4 ? kRK4S2 : kRK3S2;
-  StageArgs32 a32 = h->fp32c ? stage_args32(h, 0) : StageArgs32{};
-  a32.c1 = 0.5 * h->cfg.dt;
-  auto run = [&]() { return h->fp32c ? stage32(h, kind, a32, false) : stage(h, kind, a, false); };
   const int keep = h->tile;
-  int best = keep;
-  double best_ms = 1e300;
-  for (int v = 0; v < kTileVariants; ++v) {
-    h->tile = v;
-    int rc = run();  // warm-up (code object load, caches)
-    if (rc) { h->tile = keep; return rc; }
-    HIP_TRY(hipEventRecord(h->ev[0], h->stream));
-    for (int r = 0; r < reps; ++r)
-      if ((rc = run())) { h->tile = keep; return rc; }
-    HIP_TRY(hipEventRecord(h->ev[1], h->stream));
-    HIP_TRY(hipEventSynchronize(h->ev[1]));
-    float ms = 0.f;
-    HIP_TRY(hipEventElapsedTime(&ms, h->ev[0], h->ev[1]));
-    if (ms_per_stage) ms_per_stage[v] = ms / reps;
-    if (ms < best_ms) { best_ms = ms; best = v; }
-  }
-  h->tile = best;
-  if (tile) *tile = best;
+  const bool first = h->first_pending;
+  h->first_pending = false;  // the handed-over winds are for the first step's first stage
+  bool fused = false;
+  double ms[kTileVariants];
+  const int rc = time_shapes(
+      h->stream, h->ev, reps,
+      [&](int v) {
+        h->tile = v;
+        fused = fused_sides(h);
+        return MCV_OK;
+      },
+      [&]() {
+        const int e = rk_stage(h, kTuneStage, fused);
+        return e || fused ? e : boundary_pass(h, kTuneStage);
+      },
+      ms);
+  h->first_pending = first;
+  h->tile = rc ? keep : (int)(std::min_element(ms, ms + kTileVariants) - ms);
+  if (rc) return rc;
+  if (tile) *tile = h->tile;
+  if (ms_per_stage) std::copy(ms, ms + kTileVariants, ms_per_stage);
   return MCV_OK;
 }
 

@@ -21,6 +21,7 @@
 #pragma once
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -137,13 +138,32 @@ inline hipError_t hipGetSymbolAddress(void **p, const void *sym) {
 struct double2 {
   double x, y;
 };
-typedef void *hipEvent_t;
-inline hipError_t hipEventCreate(hipEvent_t *e) { *e = (void *)1; return hipSuccess; }
-inline hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
-inline hipError_t hipEventRecord(hipEvent_t, hipStream_t = nullptr) { return hipSuccess; }
+// Launches so far, and those of kernels named as taking raw levels; read by the
+// tests from the built library.  Time is counted in launches: an event holds
+// the count when it was recorded, and a launch lasts a millisecond.
+extern "C" {
+inline std::atomic<long> mcv_emu_launches{0}, mcv_emu_raw_launches{0};
+}
+inline void emu_count_launch(const char *kernel) {
+  ++mcv_emu_launches;
+  if (std::strstr(kernel, "raw")) ++mcv_emu_raw_launches;
+}
+typedef std::atomic<long> *hipEvent_t;
+inline hipError_t hipEventCreate(hipEvent_t *e) {
+  *e = new std::atomic<long>{0};
+  return hipSuccess;
+}
+inline hipError_t hipEventDestroy(hipEvent_t e) {
+  delete e;
+  return hipSuccess;
+}
+inline hipError_t hipEventRecord(hipEvent_t e, hipStream_t = nullptr) {
+  e->store(mcv_emu_launches);
+  return hipSuccess;
+}
 inline hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
-inline hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t) {
-  *ms = 0.f;
+inline hipError_t hipEventElapsedTime(float *ms, hipEvent_t a, hipEvent_t b) {
+  *ms = (float)(*b - *a);
   return hipSuccess;
 }
 
@@ -256,6 +276,7 @@ inline EmuTeam g_emu_team;
   do {                                                                       \
     const dim3 g_ = dim3(grid), b_ = dim3(block);                            \
     auto op_ = [=]() {                                                       \
+      emu_count_launch(#kernel);                                             \
       std::barrier<> bar_(b_.x);                                             \
       g_emu_team.run(b_.x, [&](unsigned t_) {                                \
         g_emu_block_barrier = &bar_;                                         \
@@ -279,6 +300,7 @@ inline EmuTeam g_emu_team;
   do {                                                                       \
     const dim3 g_ = dim3(grid);                                              \
     auto op_ = [=]() {                                                       \
+      emu_count_launch(#kernel);                                             \
       gridDim = g_;                                                          \
       blockDim = dim3(1);                                                    \
       threadIdx = dim3(0);                                                   \
