@@ -221,8 +221,8 @@ int mcv_batch_sync(mcv_batch *b, int32_t slot, mcv_state *out, double *mass,
 int mcv_batch_handle(mcv_batch *b, int32_t slot, mcv_handle **h);
 
 /* Times the MCV_TILE_VARIANTS tile shapes on the batch's current solves
- * (reps stage launches each, trajectory unchanged; every solve must be at a
- * step boundary) and keeps the fastest.  Blocks. */
+ * (whole stages in reps rounds, as mcv_hip_autotune; trajectory unchanged;
+ * every solve must be at a step boundary) and keeps the fastest.  Blocks. */
 int mcv_batch_autotune(mcv_batch *b, int32_t reps, int32_t *tile, double *ms_per_stage);
 
 int mcv_batch_set_tile(mcv_batch *b, int32_t tile);

@@ -374,6 +374,9 @@ struct mcv_batch {
   BatchProgress *d_prog = nullptr;
   int cur = 0;
   long long *d_stamp = nullptr;  // stages run when the boundary kernel last finished a solve
+  // the autotuner's progress tables and stamps
+  BatchProgress *d_tune_prog = nullptr;
+  long long *d_tune_stamp = nullptr;
   int *d_list = nullptr, *d_wprefix = nullptr, *d_bprefix = nullptr, *d_meta = nullptr;
   std::vector<void *> allocs;
   int variant = 0;
@@ -652,7 +655,9 @@ int mcv_batch_create(int32_t device, int32_t capacity, mcv_batch **out) {
     int rc;
     if ((rc = balloc(b, &b->d_solve, capacity)) ||
         (rc = balloc(b, &b->d_prog, 2 * (size_t)capacity)) ||
-        (rc = balloc(b, &b->d_stamp, capacity)) || (rc = balloc(b, &b->d_list, capacity)) ||
+        (rc = balloc(b, &b->d_stamp, capacity)) ||
+        (rc = balloc(b, &b->d_tune_prog, 2 * (size_t)capacity)) ||
+        (rc = balloc(b, &b->d_tune_stamp, capacity)) || (rc = balloc(b, &b->d_list, capacity)) ||
         (rc = balloc(b, &b->d_wprefix, capacity + 1)) ||
         (rc = balloc(b, &b->d_bprefix, capacity + 1)) || (rc = balloc(b, &b->d_meta, 4)))
       return rc;
@@ -779,33 +784,44 @@ int mcv_batch_autotune(mcv_batch *b, int32_t reps, int32_t *tile, double *ms_per
   HIP_TRY(hipSetDevice(b->device));
   int rc = refresh(b);
   if (rc) return rc;
-  // The first stage of every scheme reads Y_n and writes only scratch levels,
-  // the accumulator (set, not accumulated) and the band, so repeating
-  // it leaves the trajectory unchanged; it is only valid at a step boundary.
+  // only between steps is what the autotuners' stage writes free
   for (int s = 0; s < b->capacity; ++s)
     if (b->slot[s] && b->progress[s].phase != 0)
       return fail(MCV_ESTATE, "slot %d is inside a time step; autotune between steps", s);
-  const int keep = b->variant;
-  int best = keep;
-  float best_ms = 1e30f;
-  for (int v = 0; v < kTileVariants; ++v) {
-    b->variant = v;
-    if ((rc = upload_tables(b))) break;
-    if ((rc = launch_stage(b, v))) break;
-    HIP_TRY(hipEventRecord(b->ev[0], b->stream));
-    for (int r = 0; r < reps && rc == MCV_OK; ++r) rc = launch_stage(b, v);
-    if (rc) break;
-    HIP_TRY(hipEventRecord(b->ev[1], b->stream));
-    HIP_TRY(hipEventSynchronize(b->ev[1]));
-    float ms = 0.f;
-    HIP_TRY(hipEventElapsedTime(&ms, b->ev[0], b->ev[1]));
-    if (ms_per_stage) ms_per_stage[v] = ms / reps;
-    if (ms < best_ms) { best_ms = ms; best = v; }
+  // every solve with steps left at that stage, its level raw (no such stamp)
+  std::vector<BatchProgress> at(b->progress);
+  for (BatchProgress &p : at) {
+    p.phase = kTuneStage;
+    p.first = 0;
   }
-  b->variant = rc ? keep : best;
+  const std::vector<long long> stamps(b->capacity, -1);
+  HIP_TRY(hipMemcpy(b->d_tune_prog, at.data(), sizeof(BatchProgress) * b->capacity,
+                    hipMemcpyHostToDevice));
+  HIP_TRY(hipMemcpy(b->d_tune_stamp, stamps.data(), sizeof(long long) * b->capacity,
+                    hipMemcpyHostToDevice));
+  const int keep = b->variant;
+  double ms[kTileVariants];
+  std::swap(b->d_prog, b->d_tune_prog);
+  std::swap(b->d_stamp, b->d_tune_stamp);
+  rc = time_shapes(
+      b->stream, b->ev, reps,
+      [&](int v) {
+        b->variant = v;
+        return upload_tables(b);
+      },
+      [&]() {  // as run_stage, from progress table 0 each time
+        const int e = run_stage(b);
+        b->cur = 0;
+        return e;
+      },
+      ms);
+  std::swap(b->d_prog, b->d_tune_prog);
+  std::swap(b->d_stamp, b->d_tune_stamp);
+  b->variant = rc ? keep : (int)(std::min_element(ms, ms + kTileVariants) - ms);
   b->tables_dirty = true;
   if (rc) return rc;
-  if (tile) *tile = best;
+  if (tile) *tile = b->variant;
+  if (ms_per_stage) std::copy(ms, ms + kTileVariants, ms_per_stage);
   return upload_tables(b);
 }
 
