@@ -562,19 +562,31 @@ bool fused_sides(const mcv_handle *h) {
 }
 
 // nsteps time steps.  Y_n is finished when they are enqueued, as a following
-// call and the read-backs expect it.
+// call and the read-backs expect it, also where a launch fails on the way: the
+// steps whose last stage was launched count, and their level is finished from
+// that stage's band.
 int run_steps(mcv_handle *h, int32_t nsteps) {
   const int nst = stage_count(h->cfg.scheme);
-  const bool fused = fused_sides(h);
-  bool raw = false;  // the next stage's input is as a stage left it
+  const bool fused = fused_sides(h), first = h->first_pending;
+  bool raw = false;   // the next stage's input is as a stage left it
+  bool open = false;  // and so is Y_n
   for (int32_t k = 0; k < nsteps; ++k) {
     for (int s = 0; s < nst; ++s) {
+      const bool last = s == nst - 1;
       int rc = rk_stage(h, s, raw);
-      if (rc) return rc;
-      raw = fused && !(k == nsteps - 1 && s == nst - 1);
-      if (!raw && (rc = boundary_pass(h, s))) return rc;
+      if (rc == MCV_OK) {
+        if (last) ++h->steps;
+        open = open || last;
+        raw = fused && !(k == nsteps - 1 && last);
+        if (!raw && (rc = boundary_pass(h, s)) == MCV_OK) open = open && !last;
+      }
+      if (rc) {
+        const std::string msg = g_last_error;
+        if (open) (void)boundary_pass(h, nst - 1);
+        if (h->steps == 0) h->first_pending = first;  // Y_n is still what was handed over
+        return fail(rc, "%s", msg.c_str());
+      }
     }
-    ++h->steps;
   }
   return MCV_OK;
 }

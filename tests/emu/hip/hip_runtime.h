@@ -96,7 +96,17 @@ enum hipMemcpyKind {
   hipMemcpyHostToHost
 };
 inline const char *hipGetErrorString(hipError_t) { return "emulated"; }
-inline hipError_t hipGetLastError() { return hipSuccess; }
+// a test sets mcv_emu_fail_launch in the built library to n: the n-th launch from
+// then on does not run and leaves an error
+extern "C" {
+inline std::atomic<long> mcv_emu_fail_launch{0};
+}
+inline thread_local hipError_t g_emu_error = hipSuccess;
+inline hipError_t hipGetLastError() {
+  const hipError_t e = g_emu_error;
+  g_emu_error = hipSuccess;
+  return e;
+}
 inline hipError_t hipSetDevice(int) { return hipSuccess; }
 inline hipError_t hipDeviceSynchronize() { return hipSuccess; }
 inline hipError_t hipStreamCreate(hipStream_t *s) { *s = (void *)1; return hipSuccess; }
@@ -144,9 +154,14 @@ struct double2 {
 extern "C" {
 inline std::atomic<long> mcv_emu_launches{0}, mcv_emu_raw_launches{0};
 }
-inline void emu_count_launch(const char *kernel) {
+inline bool emu_launch_fails(const char *kernel) {
+  if (mcv_emu_fail_launch > 0 && --mcv_emu_fail_launch == 0) {
+    g_emu_error = 1;
+    return true;
+  }
   ++mcv_emu_launches;
   if (std::strstr(kernel, "raw")) ++mcv_emu_raw_launches;
+  return false;
 }
 typedef std::atomic<long> *hipEvent_t;
 inline hipError_t hipEventCreate(hipEvent_t *e) {
@@ -276,7 +291,7 @@ inline EmuTeam g_emu_team;
   do {                                                                       \
     const dim3 g_ = dim3(grid), b_ = dim3(block);                            \
     auto op_ = [=]() {                                                       \
-      emu_count_launch(#kernel);                                             \
+      if (emu_launch_fails(#kernel)) return;                                 \
       std::barrier<> bar_(b_.x);                                             \
       g_emu_team.run(b_.x, [&](unsigned t_) {                                \
         g_emu_block_barrier = &bar_;                                         \
@@ -300,7 +315,7 @@ inline EmuTeam g_emu_team;
   do {                                                                       \
     const dim3 g_ = dim3(grid);                                              \
     auto op_ = [=]() {                                                       \
-      emu_count_launch(#kernel);                                             \
+      if (emu_launch_fails(#kernel)) return;                                 \
       gridDim = g_;                                                          \
       blockDim = dim3(1);                                                    \
       threadIdx = dim3(0);                                                   \
