@@ -571,16 +571,21 @@ int run_stage(mcv_batch *b) {
   return b->fused ? MCV_OK : launch_boundary(b, true);
 }
 
-// The end of a run: every level finished, progress table 0 current.
-int finish_run(mcv_batch *b) {
-  int rc;
-  if (b->fused && (rc = launch_boundary(b, false))) return rc;
+// The end of a run that has come to `rc`: progress table 0 current and, where
+// the last pass is due (`pass`, or some launch failed), every level finished.
+// Also after an error, for the stages launched before it; returns the first
+// error.
+int finish_run(mcv_batch *b, int rc, bool pass) {
+  const std::string msg = rc ? mcv_hip_last_error() : "";
+  int end = pass || rc ? launch_boundary(b, false) : MCV_OK;
   if (b->cur) {
-    HIP_TRY(hipMemcpyAsync(b->d_prog, b->d_prog + b->capacity, sizeof(BatchProgress) * b->capacity,
-                           hipMemcpyDeviceToDevice, b->stream));
+    const hipError_t e =
+        hipMemcpyAsync(b->d_prog, b->d_prog + b->capacity, sizeof(BatchProgress) * b->capacity,
+                       hipMemcpyDeviceToDevice, b->stream);
     b->cur = 0;
+    if (e != hipSuccess) end = fail(MCV_EDEVICE, "progress copy: %s", hipGetErrorString(e));
   }
-  return MCV_OK;
+  return rc ? fail(rc, "%s", msg.c_str()) : end;
 }
 
 int capture(mcv_batch *b) {
@@ -727,7 +732,7 @@ int mcv_batch_run(mcv_batch *b, int32_t nstages) {
   if (!b) return fail(MCV_EINVAL, "batch is NULL");
   if (nstages < 0) return fail(MCV_EINVAL, "nstages must be >= 0");
   HIP_TRY(hipSetDevice(b->device));
-  int rc;
+  int rc = MCV_OK;
   if (b->tables_dirty && (rc = upload_tables(b))) return rc;
   int left = nstages;
   if (b->use_graph && left >= kGraphStages) {
@@ -736,12 +741,13 @@ int mcv_batch_run(mcv_batch *b, int32_t nstages) {
         b->exec_fused != b->fused) {
       if ((rc = capture(b))) return rc;
     }
-    for (; left >= kGraphStages; left -= kGraphStages)
-      HIP_TRY(hipGraphLaunch(b->exec, b->stream));
+    for (; left >= kGraphStages && rc == MCV_OK; left -= kGraphStages) {
+      const hipError_t e = hipGraphLaunch(b->exec, b->stream);
+      if (e != hipSuccess) rc = fail(MCV_EDEVICE, "hipGraphLaunch: %s", hipGetErrorString(e));
+    }
   }
-  for (; left > 0; --left)
-    if ((rc = run_stage(b))) return rc;
-  if (nstages > 0 && (rc = finish_run(b))) return rc;
+  for (; left > 0 && rc == MCV_OK; --left) rc = run_stage(b);
+  if (nstages > 0 && (rc = finish_run(b, rc, b->fused))) return rc;
   b->stages_run += nstages;
   return MCV_OK;
 }
@@ -846,17 +852,17 @@ int mcv_batch_run_timed(mcv_batch *b, int32_t nstages, double *stage_ms, double 
   if (!b) return fail(MCV_EINVAL, "batch is NULL");
   if (nstages < 0) return fail(MCV_EINVAL, "nstages must be >= 0");
   HIP_TRY(hipSetDevice(b->device));
-  int rc;
+  int rc = MCV_OK;
   if (b->tables_dirty && (rc = upload_tables(b))) return rc;
   double sm = 0.0, bm = 0.0;
-  // the boundary pass after each stage, or after the last one
-  for (int i = 0; i < nstages; ++i) {
-    const bool pass = !b->fused || i == nstages - 1;
+  // one stage and, after each stage or after the last one, the boundary pass
+  auto timed = [&](bool pass) -> int {
+    int e;
     HIP_TRY(hipEventRecord(b->ev[0], b->stream));
-    if ((rc = launch_stage(b, b->variant))) return rc;
+    if ((e = launch_stage(b, b->variant))) return e;
     b->cur = 1 - b->cur;
     HIP_TRY(hipEventRecord(b->ev[1], b->stream));
-    if (pass && (rc = launch_boundary(b, !b->fused))) return rc;
+    if (pass && (e = launch_boundary(b, !b->fused))) return e;
     HIP_TRY(hipEventRecord(b->ev[2], b->stream));
     HIP_TRY(hipEventSynchronize(b->ev[2]));
     float a = 0.f, c = 0.f;
@@ -864,12 +870,10 @@ int mcv_batch_run_timed(mcv_batch *b, int32_t nstages, double *stage_ms, double 
     HIP_TRY(hipEventElapsedTime(&c, b->ev[1], b->ev[2]));
     sm += a;
     if (pass) bm += c;
-  }
-  if (nstages > 0 && b->cur) {
-    HIP_TRY(hipMemcpyAsync(b->d_prog, b->d_prog + b->capacity, sizeof(BatchProgress) * b->capacity,
-                           hipMemcpyDeviceToDevice, b->stream));
-    b->cur = 0;
-  }
+    return MCV_OK;
+  };
+  for (int i = 0; i < nstages && rc == MCV_OK; ++i) rc = timed(!b->fused || i == nstages - 1);
+  if (nstages > 0 && (rc = finish_run(b, rc, false))) return rc;
   b->stages_run += nstages;
   if (stage_ms) *stage_ms = sm;
   if (boundary_ms) *boundary_ms = bm;

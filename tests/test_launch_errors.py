@@ -1,7 +1,7 @@
 """A launch that fails in the middle of a call (CPU emulation: the n-th launch of
-a call does not run and reports an error): the call says so, the steps that were
-completed before it count, what is read back is the state after them, bit for
-bit, and the solve goes on from there."""
+a call does not run and reports an error): the call says so, the steps (in a
+batch, stages) that were completed before it count, what is read back is the
+state after them, bit for bit, and the solve goes on from there."""
 import ctypes
 
 import numpy as np
@@ -55,3 +55,53 @@ def test_emulated_step_goes_on_after_a_failed_launch(emu_lib, scheme, precision,
             assert _same(s.sync(), ref[done], ok), f
             s.step(STEPS + MORE - done)
             assert _same(s.sync(), ref[-1], ok), f
+
+
+@pytest.mark.parametrize("tile", [0, 1])
+@pytest.mark.parametrize("timed", [False, True])
+def test_emulated_batch_goes_on_after_a_failed_launch(emu_lib, timed, tile):
+    specs = [(3, 5, "RK3_TVD", capi.FP32C, 5), (4, 3, "RK4", capi.FP64, 4)]
+
+    def batch():
+        b = capi.Batch(3, lib=emu_lib)
+        slots = []
+        for dof, n, scheme, precision, steps in specs:
+            m = cases.mesh(dof, n)
+            slots.append(b.add(dof, n, 200.0, m, cases.case5(m), steps, scheme=scheme,
+                               precision=precision))
+        b.set_tile(tile)
+        return b, slots
+
+    def same(b, slots, ref):
+        for (dof, n, *_), slot, r in zip(specs, slots, ref):
+            assert _same(b.sync(slot), r, cases.masks(dof, n)["defined"])
+
+    b, slots = batch()
+    with b:
+        b.run(16)
+        ref = [b.sync(s) for s in slots]
+    stages = 5
+    # the launch that fails: a stage or a boundary pass, at either progress table
+    for f in range(1, (stages if tile == 0 else 2 * stages) + 1):
+        b, slots = batch()
+        with b:
+            _fail_launch(emu_lib, f)
+            with pytest.raises(capi.MCVError) as e:
+                b.run_timed(stages) if timed else b.run(stages)
+            assert e.value.code == capi.MCV_EDEVICE
+            done = f - 1 if tile == 0 else f // 2  # stages launched
+            left, steps = b.poll()
+            assert list(steps[:2]) == [done // 3, done // 4], f
+            # a solve admitted now is not taken from an older table
+            extra = b.add(3, 5, 200.0, *_inputs(), 1)
+            b.run(12 - done)  # to a step boundary of both
+            left, steps = b.poll()
+            assert list(steps) == [4, 3, 1] and list(left) == [1, 1, 0], f
+            b.run(12)  # a graph where graphs are used
+            same(b, slots, ref)
+            assert np.isfinite(b.sync(extra)["mass"])
+
+
+def _inputs():
+    m = cases.mesh(3, 5)
+    return m, cases.case5(m)
