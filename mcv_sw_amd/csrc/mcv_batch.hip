@@ -429,6 +429,7 @@ void destroy_batch(mcv_batch *b) {
   for (void *p : b->allocs) (void)hipFree(p);
   if (b->stream) (void)hipStreamDestroy(b->stream);
   delete b;
+  staging_user(-1);
 }
 
 BatchSolve describe(const mcv_handle *h) {
@@ -648,6 +649,7 @@ int mcv_batch_create(int32_t device, int32_t capacity, mcv_batch **out) {
     return fail(MCV_EINVAL, "capacity must be in [1, 65536], got %d", capacity);
   mcv_batch *b = new (std::nothrow) mcv_batch();
   if (!b) return fail(MCV_ENOMEM, "host allocation failed");
+  staging_user(1);  // until destroy_batch: kept from one admission to the next
   auto init = [&]() -> int {
     b->device = device;
     b->capacity = capacity;

@@ -15,6 +15,9 @@ namespace mcv {
 
 // Records the message returned by mcv_hip_last_error() and returns code.
 int fail(int code, const char *fmt, ...);
+// A solve or a batch comes (1) or goes (-1): the read-backs' pinned memory is
+// given back with the last of them (mcv_hip.hip).
+void staging_user(int change);
 // mcv_history_write that also checks the file's per-record sizes (mcv_netcdf.cpp)
 int history_write_checked(const char *path, int32_t time_slot, const mcv_history_fields *rec,
                           long long npoint, long long ncell);

@@ -155,13 +155,14 @@ char *scratch_of(int device) {
 //
 // The pinned slots (32 MB) and events serve one call at a time (another call
 // at the same moment, or on another device, takes the plain copy), are made by
-// the first such read-back and given back with the last handle.
+// the first such read-back and given back with the last solve or batch.
 constexpr size_t kStagedBytes = size_t(4) << 20, kManyBytes = size_t(24) << 20;
 constexpr size_t kSlotBytes = size_t(2) << 20;
 constexpr int kCopyThreads = 8;
 struct Staging {
-  std::mutex mu;
-  int handles = 0;  // live handles
+  std::mutex users_mu;
+  int users = 0;  // live solves and batches
+  std::mutex mu;  // held by the read-back that uses what follows
   int device = -1;
   char *slots = nullptr;  // 2 per copy thread
   hipEvent_t ev[2 * kCopyThreads] = {};
@@ -188,15 +189,24 @@ bool staging_ready(Staging &g, int device) {
   return true;
 }
 
-void staging_handle(int change) {
-  std::lock_guard<std::mutex> lock(g_staging.mu);
+}  // namespace
+
+// A solve or a batch comes or goes.  Whoever takes the slots for a copy belongs
+// to one of them, so the last to go finds them idle; the others do not wait for
+// a copy that is running.
+void mcv::staging_user(int change) {
   Staging &g = g_staging;
-  g.handles += change;
-  if (g.handles > 0 || !g.slots) return;
+  std::lock_guard<std::mutex> users(g.users_mu);
+  g.users += change;
+  if (g.users > 0) return;
+  std::lock_guard<std::mutex> lock(g.mu);
+  if (!g.slots) return;
   for (hipEvent_t e : g.ev) (void)hipEventDestroy(e);
   (void)hipHostFree(g.slots);
   g.slots = nullptr;
 }
+
+namespace {
 
 struct Download {
   void *dst;
@@ -328,7 +338,7 @@ void destroy(mcv_handle *h) {
     if (e) (void)hipEventDestroy(e);
   for (void *p : h->allocs) (void)hipFree(p);
   delete h;
-  staging_handle(-1);
+  staging_user(-1);
 }
 
 int validate(const mcv_config *c) {
@@ -970,7 +980,7 @@ int mcv_hip_init(const mcv_config *cfg, const mcv_mesh *mesh, const mcv_state *i
   *out = nullptr;
   mcv_handle *h = new (std::nothrow) mcv_handle();
   if (!h) return fail(MCV_ENOMEM, "host allocation failed");
-  staging_handle(1);  // until destroy
+  staging_user(1);  // until destroy
   int rc = init_impl(cfg, mesh, initial, h);
   if (rc) {
     std::string msg = g_last_error;

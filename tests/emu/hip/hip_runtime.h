@@ -117,8 +117,19 @@ inline hipError_t hipMalloc(void **p, size_t n) {
   return *p ? hipSuccess : 2;
 }
 inline hipError_t hipFree(void *p) { std::free(p); return hipSuccess; }
-inline hipError_t hipHostMalloc(void **p, size_t n, unsigned) { return hipMalloc(p, n); }
-inline hipError_t hipHostFree(void *p) { return hipFree(p); }
+// pinned allocations made and not yet freed, read by the tests
+extern "C" {
+inline std::atomic<long> mcv_emu_pinned_made{0}, mcv_emu_pinned_live{0};
+}
+inline hipError_t hipHostMalloc(void **p, size_t n, unsigned) {
+  ++mcv_emu_pinned_made;
+  ++mcv_emu_pinned_live;
+  return hipMalloc(p, n);
+}
+inline hipError_t hipHostFree(void *p) {
+  --mcv_emu_pinned_live;
+  return hipFree(p);
+}
 inline hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind) {
   std::memcpy(d, s, n);
   return hipSuccess;

@@ -3,6 +3,7 @@ a time (plain copies): the same bytes, also with two solves read at once (one
 of them finds the copy threads busy).  Sizes on both sides of the rule: six
 fields of 1.7 MB (four threads) and of 7 MB (eight), none a whole number of
 chunks."""
+import ctypes
 import threading
 
 import numpy as np
@@ -42,6 +43,27 @@ def test_emulated_large_readback(emu_lib, dof, n):
         out = s.sync(integrals=False)
         for k in capi.STATE_FIELDS:
             assert np.array_equal(out[k], s.sync(fields=(k,), integrals=False)[k]), k
+
+
+def test_emulated_pinned_memory_is_kept_by_a_batch(emu_lib):
+    """One solve at a time through a resident batch: the pinned memory of the
+    read-backs is made once, and given back with the batch."""
+    lib = ctypes.CDLL(emu_lib)
+
+    def pinned(name):
+        return ctypes.c_long.in_dll(lib, f"mcv_emu_pinned_{name}").value
+
+    m = cases.mesh(4, 60)
+    st = cases.case5(m)
+    made = pinned("made")
+    with capi.Batch(1, lib=emu_lib) as b:
+        for _ in range(3):
+            slot = b.add(4, 60, 50.0, m, st, 0)
+            out = b.sync(slot, integrals=False)
+            assert np.array_equal(out["phi"], st["phi"])
+            b.remove(slot)
+        assert pinned("made") == made + 1 and pinned("live") == 1
+    assert pinned("live") == 0
 
 
 @pytest.mark.gpu
