@@ -155,7 +155,8 @@ def test_tsan_build_finds_no_race_within_a_block():
     under ThreadSanitizer: no two threads of a block touch the same LDS or
     global word without a __syncthreads() between them, in any stage kind,
     tile shape, boundary, diagnostic or batched kernel (a removed barrier in
-    the stage kernel is reported as a data race by this build)."""
+    the stage kernel is reported as a data race by this build); nor do the copy
+    threads of a large read-back."""
     sys.path.insert(0, os.path.join(ROOT, "tests", "emu"))
     import build_emu
 

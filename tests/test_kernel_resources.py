@@ -8,7 +8,9 @@ product's flags).  Compiles on the CPU; no GPU needed.
   - the FP64 MCV4 single-solve stage kernels at the 6x4 and 5x5 cell tiles
     (the shapes the autotuner takes at 6x384^2, whose LDS, 27-28 KB, allows
     5 workgroups per CU) stay within 80 VGPRs and run at least 5 waves per
-    SIMD.
+    SIMD;
+  - the kernels that run the boundary pass inside, single-solve and batched,
+    reach the waves per SIMD they are compiled for (stage_waves, batch_waves).
 """
 import os
 import re
@@ -71,6 +73,40 @@ def test_fp64_stage_kernels_within_80_vgprs(kernels):
             if re.match(r"_ZN3mcv12stage_kernelILi4ELi\dELi(6ELi4|5ELi5)E", k)}
     assert len(fp64) == 8 * 2  # stage kinds (tendency + 7) x tile shapes
     assert all(v["vgpr"] <= 80 and v["occupancy"] >= 5 for v in fp64.values()), fp64
+
+
+# waves per SIMD of stage_kernel_raw at tile shapes 0 and 2 of (form, order)
+RAW_WAVES = {("", 3): {"8,7": 6, "10,5": 6}, ("", 4): {"6,4": 6, "5,5": 5},
+             ("_f32", 3): {"8,7": 8, "10,5": 8}, ("_f32", 4): {"6,4": 8, "8,8": 4}}
+
+
+def test_raw_stage_kernels_reach_their_waves(kernels):
+    seen = 0
+    for name, v in kernels.items():
+        m = re.match(r"_ZN3mcv\d+stage_kernel_raw(_f32)?ILi(\d)ELi\dELi(\d+)ELi(\d+)E", name)
+        if m:
+            want = RAW_WAVES[(m[1] or "", int(m[2]))][f"{m[3]},{m[4]}"]
+            assert v["occupancy"] >= want, (name, v)
+            seen += 1
+    assert seen == 8 * 7  # shapes of both orders and forms x stage kinds
+
+
+# of batch_raw_stage_kernel: bodies (FP64 MCV3 1, MCV4 2, FP32C MCV3 4, MCV4 8) ->
+# at shape 0, at shape 2, and at shape 0 and 2 with both schemes in one kernel
+BATCH_RAW_WAVES = {1: (6, 6, 6, 6), 2: (5, 5, 5, 5), 4: (8, 8, 6, 6), 8: (8, 4, 6, 4),
+                   3: (5, 4, 5, 4), 12: (8, 4, 6, 4), 15: (5, 4, 5, 4)}
+
+
+def test_raw_batch_kernels_reach_their_waves(kernels):
+    seen = 0
+    for name, v in kernels.items():
+        m = re.match(r"_ZN3mcv\d+batch_raw_stage_kernelILi(\d)ELi(\d+)E", name)
+        if m:
+            shape, mask = int(m[1]), int(m[2])
+            col = (0 if shape == 0 else 1) + (2 if mask >> 4 == 3 else 0)
+            assert v["occupancy"] >= BATCH_RAW_WAVES[mask & 15][col], (name, v)
+            seen += 1
+    assert seen == 2 * 21
 
 
 def test_div_small_exact_on_its_domain():

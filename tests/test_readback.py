@@ -1,8 +1,8 @@
-"""Large read-backs through the copy threads against single fields read one at
-a time (plain copies): the same bytes, also with two solves read at once (one
-of them finds the copy threads busy).  Sizes on both sides of the rule: six
-fields of 1.7 MB (four threads) and of 7 MB (eight), none a whole number of
-chunks."""
+"""Large read-backs through the copy threads against the handed-over state, which
+a solve holds until its first step: the same bytes, also with two solves read at
+once (one of them finds the copy threads busy).  Sizes on both sides of the rule:
+six fields of 1.7 MB (four threads) and of 7 MB (eight), none a whole number of
+chunks; single fields below the rule (a plain copy) and above it."""
 import ctypes
 import threading
 
@@ -13,12 +13,23 @@ import cases
 from mcv_sw_amd import capi
 
 
+def _handed_over(m, st):
+    return {**{k: st[k] for k in capi.STATE_FIELDS}, "phiG": st["phi"] * m["sqrtG"]}
+
+
+def _assert_same(out, want):
+    for k, x in out.items():
+        assert np.array_equal(x, want[k]), k
+
+
 def _check(lib, dof, n):
     m = cases.mesh(dof, n)
     st = cases.case5(m)
+    want = _handed_over(m, st)
     with capi.Solver(dof, n, 50.0, m, st, lib=lib) as a, capi.Solver(dof, n, 50.0, m, st,
                                                                      lib=lib) as b:
-        one = {k: a.sync(fields=(k,), integrals=False)[k] for k in capi.STATE_FIELDS}
+        for k in capi.STATE_FIELDS:
+            _assert_same(a.sync(fields=(k,), integrals=False), want)
         outs = [None, None]
 
         def read(i, s):
@@ -30,8 +41,8 @@ def _check(lib, dof, n):
         for t in team:
             t.join()
         for out in outs[0] + outs[1]:
-            for k in capi.STATE_FIELDS:
-                assert np.array_equal(out[k], one[k]), k
+            assert set(out) == set(capi.STATE_FIELDS)
+            _assert_same(out, want)
 
 
 @pytest.mark.parametrize("dof,n", [(4, 60), (3, 190)])
@@ -39,10 +50,11 @@ def test_emulated_large_readback(emu_lib, dof, n):
     # one solve at a time here: the shim's launches share their LDS statics
     m = cases.mesh(dof, n)
     st = cases.case5(m)
+    want = _handed_over(m, st)
     with capi.Solver(dof, n, 50.0, m, st, lib=emu_lib) as s:
-        out = s.sync(integrals=False)
+        _assert_same(s.sync(integrals=False), want)
         for k in capi.STATE_FIELDS:
-            assert np.array_equal(out[k], s.sync(fields=(k,), integrals=False)[k]), k
+            _assert_same(s.sync(fields=(k,), integrals=False), want)
 
 
 def test_emulated_pinned_memory_is_kept_by_a_batch(emu_lib):
