@@ -266,8 +266,13 @@ constexpr bool eight_waves(int V, int M) {
 }
 
 // Waves per SIMD of the raw builds (the boundary pass would take registers
-// freely, see stage_waves): eight_waves' choice, else those of the bodies' single-solve kernels,
-// one less where a kernel holds several bodies (whose tables take registers too).
+// freely, see stage_waves): eight_waves' choice, else those of the bodies'
+// single-solve kernels, one less where a kernel holds several bodies (whose
+// tables take registers too), and two limits.  5 with the FP64 MCV4 body: asked
+// for 6 it spills 2 to 12 VGPRs to scratch memory.  6 for the rest, which leaves
+// FP32C with both schemes 7 waves; asked for 8, us per stage of two or four
+// solves at 6 / at 8: MCV3 6x64^2 12.1 / 12.4, 6x90^2 28.7 / 27.0, MCV4 6x45^2
+// 23.0 / 21.7, 6x90^2 30.1 / 29.1 (56 to 83 spilled scalars at 8).
 template <int V>
 constexpr int batch_waves_v(int M) {
   int w = 8;

@@ -247,7 +247,7 @@ __device__ __forceinline__ void stage_body_f32(const MeshF32 &m, const StageArgs
   else stage_points(std::false_type{});
   __syncthreads();
 
-  // cell ends: a wavefront works along one direction (see stage_tile)
+  // cell ends: a wavefront works along one direction (see stage_body)
   constexpr int kTasksX = (CX + 1) * NY, kTasksY = (CY + 1) * NX;
   constexpr int kStartY = (kTasksX + 63) / 64 * 64;
   auto cell_end = [&](auto xdir, const int tt) {
@@ -316,7 +316,7 @@ __device__ __forceinline__ void stage_body_f32(const MeshF32 &m, const StageArgs
   }
   __syncthreads();
 
-  // owned points row by row (see stage_tile); global loads of all a thread's
+  // owned points row by row (see stage_body); global loads of all a thread's
   // points first, then their LDS work
   constexpr int kRow = CX * H, kSlots = kRow * CY * H, kTail = NY + NX - 1;
   constexpr int kP2 = (kSlots + kTail + kStageThreads - 1) / kStageThreads;
