@@ -79,9 +79,23 @@ def fp32c_bytes_per_point_step(scheme):
     return 36 + 24 + 12 + 36 + 12 + 3 * 24
 
 
-def measured_traffic(path):
+def stage_source():
+    """Digest of the FP64 stage kernel's sources, comments and spacing left out:
+    a profile names the one it was taken from."""
+    import hashlib
+    import re
+
+    h = hashlib.sha256()
+    for f in ("mcv_device.hpp", "mcv_halo.hpp", "mcv_stage_fp64.hpp"):
+        text = open(os.path.join(ROOT, "mcv_sw_amd", "csrc", f)).read()
+        h.update(re.sub(r"\s+", " ", re.sub(r"//[^\n]*", "", text)).encode())
+    return h.hexdigest()[:16]
+
+
+def measured_traffic(path, tile):
     """Calibrated HBM bytes per stage launch from the committed rocprofv3
-    FETCH_SIZE/WRITE_SIZE summary (profiles/), or None."""
+    FETCH_SIZE/WRITE_SIZE summary (profiles/); None without one of the present
+    kernel at this tile shape."""
     import re
 
     try:
@@ -89,7 +103,9 @@ def measured_traffic(path):
     except OSError:
         return None
     m = re.search(r"Per RK4 step: (\d+(?:\.\d+)?) MB measured", text)
-    return float(m.group(1)) * 1e6 / 4 if m else None
+    if not m or f"Stage kernel source: {stage_source()}, tile shape {tile}" not in text:
+        return None
+    return float(m.group(1)) * 1e6 / 4
 
 
 def owned(a, dof, n):
@@ -504,7 +520,8 @@ def main():
     bytes_per_launch = bpcs * cells / 4
     avg_launch_s = rec64["stage_kernel_ms_per_step"] / 4 / 1e3
     achieved = bytes_per_launch / avg_launch_s / 1e9
-    traffic = measured_traffic(os.path.join(ROOT, "profiles", "stage_kernel_mcv4_n384_fp64.md"))
+    traffic = measured_traffic(os.path.join(ROOT, "profiles", "stage_kernel_mcv4_n384_fp64.md"),
+                               rec64["tile_variant"])
     res = {
         "metric": "SW cell-steps/s (plain FP64 vs batched FP32) at stated h err; serve p50/p99",
         "value": rec64["value"],

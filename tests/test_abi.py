@@ -171,3 +171,17 @@ def test_bench_refuses_more_than_one_gpu():
                        capture_output=True, text=True, timeout=120)
     assert p.returncode == 2
     assert "one GPU" in p.stderr
+
+
+def test_bench_reports_traffic_of_the_present_kernel_only(tmp_path):
+    sys.path.insert(0, ROOT)
+    import bench
+
+    def reported(source, tile):
+        f = tmp_path / "profile.md"
+        f.write_text(f"Stage kernel source: {source}, tile shape 2\nPer RK4 step: 4000.0 MB measured\n")
+        return bench.measured_traffic(str(f), tile)
+
+    assert reported(bench.stage_source(), 2) == 1e9
+    assert reported("0" * 16, 2) is None
+    assert reported(bench.stage_source(), 0) is None
