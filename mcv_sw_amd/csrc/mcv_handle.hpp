@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <vector>
 
@@ -109,19 +110,21 @@ BoundaryArgs32 boundary_args32(const mcv_handle *h, int s);
 // Milliseconds per stage of every tile shape: use(v) switches to shape v,
 // stage() enqueues a stage as the steps would run it, boundary launch included
 // where the shape needs one.  The shapes take turns, `reps` rounds, so that a
-// drift meets them all; each turn is timed over at least kTuneMs (a stretch of
-// three stages of 7 us told shapes 5% apart wrongly) behind a stage that is not,
-// and the best turn counts.
-constexpr float kTuneMs = 0.25f;
+// drift meets them all; a turn is timed behind a stage that is not, over about
+// kTuneMs (at most kTuneStages), and the best turn counts.  A shape that is a
+// fifth behind after a round is not tried again.
+constexpr float kTuneMs = 0.1f;
+constexpr int kTuneStages = 8;
 template <class Use, class Stage>
 int time_shapes(hipStream_t stream, hipEvent_t *ev, int reps, const Use &use, const Stage &stage,
                 double *ms) {
-  int stages[kTileVariants];
-  for (int r = -1; r < reps; ++r)  // the first round sets the stretches (and loads the code)
+  int stages[kTileVariants] = {1, 1, 1, 1};
+  static_assert(kTileVariants == 4, "one entry per shape");
+  for (int r = -1; r < reps; ++r)  // the first round loads the code and sets the stretches
     for (int v = 0; v < kTileVariants; ++v) {
-      const int n = r < 0 ? 1 : stages[v];
+      if (r > 0 && ms[v] > 1.2 * *std::min_element(ms, ms + kTileVariants)) continue;
       int rc = use(v);
-      for (int k = 0; k <= n && rc == MCV_OK; ++k) {
+      for (int k = 0; k <= stages[v] && rc == MCV_OK; ++k) {
         if (k == 1) HIP_TRY(hipEventRecord(ev[0], stream));
         rc = stage();
       }
@@ -130,8 +133,9 @@ int time_shapes(hipStream_t stream, hipEvent_t *ev, int reps, const Use &use, co
       HIP_TRY(hipEventSynchronize(ev[1]));
       float t = 0.f;
       HIP_TRY(hipEventElapsedTime(&t, ev[0], ev[1]));
-      if (r < 0) stages[v] = t * 16 < kTuneMs ? 16 : 1 + (int)(kTuneMs / t);
-      else if (r == 0 || t / n < ms[v]) ms[v] = t / n;
+      t /= stages[v];
+      ms[v] = r <= 0 ? t : std::min(ms[v], (double)t);
+      if (r < 0) stages[v] = t * kTuneStages < kTuneMs ? kTuneStages : 1 + (int)(kTuneMs / t);
     }
   return MCV_OK;
 }
